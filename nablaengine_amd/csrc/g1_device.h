@@ -378,15 +378,15 @@ __device__ __forceinline__ void cross(const float* a, const float* b, float* o) 
 __device__ __forceinline__ float dot3(const float* a, const float* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
 // ------------------------------------------------------------------------------------------------ LTL factorization
-// A = L' L with L lower triangular, eliminated leaf-first (k = NV-1 .. 0), as MuJoCo factors M: with parents before
-// children in the dof order, row k of L is nonzero only at k's ancestor dofs (no fill-in) for a matrix with the
-// tree's sparsity (M, and H = M + J'DJ when no contact couples two robot bodies). Lane j holds column j of the lower
-// triangle in registers (c[m] = A[m][j], m >= j), so row k's entries L[k][j] are lane-local and L[k][m] is one
-// v_readlane away: step k is one pivot and, per ancestor m of k, a broadcast and one FMA on every lane.
-// SPARSE = false visits every m < k (the dense factor of a matrix with cross-branch entries). In place in Lp (packed
-// lower, TRI layout, followed by the 64-float sink at LSINK). Lane j's registers c[m] for m < j hold other entries of the matrix (loaded from in-bounds
-// addresses, not zeroed): they are updated from one another only, never broadcast (a broadcast reads lane m's c[k],
-// k > m) and never stored, so the valid entries do not depend on them.
+// The factorization for a matrix with entries across the tree's branches, H with active contacts between two robot
+// bodies (the tree's own sparsity is factored in the path layout, g1_path.h). A = L' L with L lower triangular,
+// eliminated leaf-first (k = NV-1 .. 0), as MuJoCo factors M: with parents before children in the dof order, row k of
+// L is nonzero only at k's ancestor dofs and the columns its contacts fill. Lane j holds column j of the lower triangle
+// in registers (c[m] = A[m][j], m >= j), so row k's entries L[k][j] are lane-local and L[k][m] is one v_readlane away:
+// step k is one pivot and, per column m it has, a broadcast and one FMA on every lane. In place in Lp (packed lower, TRI
+// layout, followed by the 64-float sink at LSINK). Lane j's registers c[m] for m < j hold other entries of the matrix
+// (loaded from in-bounds addresses, not zeroed): they are updated from one another only, never broadcast (a broadcast
+// reads lane m's c[k], k > m) and never stored, so the valid entries do not depend on them.
 // The fill that contacts between robot bodies of the common kinds add to the tree's sparsity: a leg against the
 // waist or its own arm, or the two legs. H gains entries between the non-shared dofs of the two chains, and
 // eliminating leaf-first spreads them to the rows of the later (higher) chain and of the shared ancestors in
@@ -403,61 +403,17 @@ __host__ __device__ constexpr uint64_t fill_bits(int k) {
 static_assert(NV == 35, "the fill rows are the G1's dof ranges");
 static_assert(NV * (NV - 1) / 2 + 63 < LSINK + 64, "the unmasked row stores of the last row stay in the factor buffer");
 
-// The hinge dofs are eliminated first; each would update the 6 x 6 root block (rows and columns 0..5) by the outer
-// product of its row's root part, 6 broadcasts and FMAs a step that only lanes 0..5 use (174 of the tree pattern's 306
-// pairs). These updates are summed instead as one product on the matrix cores, the Schur complement
-// D = X' X with X[k][r] = L[k][r] (hinge rows k = 6..34, root columns r < 6; 29 rows padded to 32): 8 steps of
-// v_mfma_f32_16x16x4f32, lane l giving A[l % 16][k'] = B[k'][l % 16] = X[6 + k'][l % 16] for k' = 4 t + l / 16 (read
-// back from the factor's hinge rows, stored first), lane l holding D[4 (l / 16) + e][l % 16]. Then the root block is
-// eliminated as before.
-// The elimination order. Any order that eliminates a dof after all its descendants gives the same factor; for the
-// tree's pattern the four branches below the root and waist (right arm 34..28, left arm 27..21, right leg 17..12, left
-// leg 11..6) are independent chains, interleaved two at a time so that consecutive steps do not wait on each other;
-// then the waist (20..18) and the root (5..0). With the self-contact fill (rows 18..27 and 12..17 gain leg columns) and
-// dense, the descending order.
 typedef float mfma4 __attribute__((ext_vector_type(4)));
 constexpr int NROOT = 6;  // the free joint's dofs: every other dof's ancestors
-struct Order { int v[NV]; };
-constexpr Order elim_order(bool tree) {
-  Order o{};
-  int n = 0;
-  if (tree) {
-    for (int t = 0; t < 7; t++) { o.v[n++] = 34 - t; o.v[n++] = 27 - t; }
-    for (int t = 0; t < 6; t++) { o.v[n++] = 17 - t; o.v[n++] = 11 - t; }
-    for (int k = 20; k >= 18; k--) o.v[n++] = k;
-    for (int k = NROOT - 1; k >= 0; k--) o.v[n++] = k;
-  } else {
-    for (int k = NV - 1; k >= 0; k--) o.v[n++] = k;
-  }
-  return o;
-}
-constexpr bool order_ok(const Order& o) {  // a permutation, each dof after all of its descendants (tree pattern)
-  bool seen[NV] = {};
-  for (int s = 0; s < NV; s++) {
-    const int k = o.v[s];
-    if (k < 0 || k >= NV || seen[k]) return false;
-    for (int d = k + 1; d < NV; d++)
-      if (((TREE.dofanc[d] >> k) & 1ull) && !seen[d]) return false;
-    seen[k] = true;
-  }
-  return true;
-}
-static_assert(order_ok(elim_order(true)) && order_ok(elim_order(false)), "elimination orders");
-static_assert(((TREE.dofanc[34] >> 18) & 1) != 0 && ((TREE.dofanc[27] >> 18) & 1) != 0 &&
-              ((TREE.dofanc[27] >> 28) & 1) == 0 && ((TREE.dofanc[17] >> 6) & 1) == 0,
-              "the G1's branches: arms 21..27 / 28..34 below the waist, legs 6..11 / 12..17");
-
 // The hinge dofs are eliminated first; each would update the 6 x 6 root block (rows and columns 0..5) by the outer
-// product of its row's root part, 6 broadcasts and FMAs a step that only lanes 0..5 use (174 of the tree pattern's 306
-// pairs). These updates are summed instead as one product on the matrix cores, the Schur complement
+// product of its row's root part, 6 broadcasts and FMAs a step that only lanes 0..5 use (174 pairs). These updates are summed instead as one product on the matrix cores, the Schur complement
 // D = X' X with X[k][r] = L[k][r] (hinge rows k = 6..34, root columns r < 6; 29 rows padded to 32): 8 steps of
 // v_mfma_f32_16x16x4f32, lane l giving A[l % 16][k'] = B[k'][l % 16] = X[6 + k'][l % 16] for k' = 4 t + l / 16 (read
 // back from the factor's hinge rows, stored first), lane l holding D[4 (l / 16) + e][l % 16]. Then the root block is
 // eliminated as before.
-template <int PATTERN>  // 0: the tree's sparsity; 1: with the common self-contact fill; 2: every pair
+template <int PATTERN>  // 1: the tree's sparsity with the common self-contact fill; 2: every pair
 __device__ __forceinline__ void ltl_factor(float* Lp, int lane_) {
   constexpr bool SPARSE = PATTERN < 2;
-  constexpr Order ORD = elim_order(PATTERN == 0);
   const int lane = opaque_lane(lane_);
   // column j = lane of the lower triangle: A[m][j] = col[tri(m, 0)] for m >= j; every lane's address inside the
   // matrix (lanes past the column select 0), all the loads issued before the elimination
@@ -465,8 +421,8 @@ __device__ __forceinline__ void ltl_factor(float* Lp, int lane_) {
   float c[NV];
 #pragma unroll
   for (int m = 0; m < NV; m++) c[m] = col[tri(m, 0)];
-  static_for<0, NV, 1>([&](auto sc) {
-    constexpr int k = ORD.v[decltype(sc)::value];
+  static_for<NV - 1, -1, -1>([&](auto kc) {
+    constexpr int k = decltype(kc)::value;
     if constexpr (k == NROOT - 1) {
       // the hinge rows are final: store them, row m at tri(m, 0) + lane on every lane, rows in increasing order. A
       // lane past the row (lane > m, or no column) writes into a later row's slots, which that row's own store
@@ -502,10 +458,10 @@ __device__ __forceinline__ void ltl_factor(float* Lp, int lane_) {
     float bc[NV];
 #pragma unroll
     for (int m = m0; m < k; m++)
-      if (!SPARSE || (((TREE.dofanc[k] | (PATTERN ? fill_bits(k) : 0ull)) >> m) & 1ull)) bc[m] = rdl(c[k], m);
+      if (!SPARSE || (((TREE.dofanc[k] | fill_bits(k)) >> m) & 1ull)) bc[m] = rdl(c[k], m);
 #pragma unroll
     for (int m = m0; m < k; m++)  // A[m][j] -= L[k][j] L[k][m] (the pattern's test at compile time)
-      if (!SPARSE || (((TREE.dofanc[k] | (PATTERN ? fill_bits(k) : 0ull)) >> m) & 1ull)) c[m] = fmaf(-c[k], bc[m], c[m]);
+      if (!SPARSE || (((TREE.dofanc[k] | fill_bits(k)) >> m) & 1ull)) c[m] = fmaf(-c[k], bc[m], c[m]);
   });
   // lane j stores column j's root rows m >= j; the other lanes store into their sink slot (the hinge rows are stored
   // already: no write past a root row may reach them)

@@ -25,17 +25,56 @@
 
 namespace g1k {
 
-// factor the packed matrix in s.L in place as L' L; dense when a contact couples two robot bodies (cross-branch
-// entries), else with the tree's sparsity
-// pattern: 0 the tree's sparsity, 1 with the common self-contact fill, 2 dense (hessian()'s classification)
-__device__ __forceinline__ void factor_L(Sim& s, int lane, int pattern = 0) {
+// factor the packed matrix in s.L in place as L' L for entries across the tree's branches: pattern 1 the tree's
+// sparsity with the common self-contact fill, 2 dense (hessian()'s classification; 0, the tree's: path_factor)
+__device__ __forceinline__ void factor_L(Sim& s, int lane, int pattern) {
 #ifdef G1_PROFILE
-  if (pattern != 0 && lane == 0) s.prof_acc[PH_DENSE] += 1;
+  if (lane == 0) s.prof_acc[PH_DENSE] += 1;
 #endif
-  if (pattern == 0) ltl_factor<0>(s.L, lane);
-  else if (pattern == 1) ltl_factor<1>(s.L, lane);
+  if (pattern == 1) ltl_factor<1>(s.L, lane);
   else ltl_factor<2>(s.L, lane);
   wsync();
+}
+
+// the lanes that hold row M's entries of a lower triangle in the path layout, each entry once
+template <int M>
+struct PathEntry {
+  static constexpr LaneMask m = lane_mask([](int g, int p) { return p <= M && path_owner(g, M); });
+};
+// packed position of entry (row m of this lane's path, column pd), m's dof being m + its row's offset
+template <int M>
+__device__ __forceinline__ int path_packed(int pd, int lane) {
+  const int g = lane >> 4, i = M + (M < 6 ? 0 : M < 9 ? (g < 2 ? 6 * g : 12) : (g < 3 ? 6 * g : 19));
+  return i * (i + 1) / 2 + pd;
+}
+// a lower triangle in the path layout (lane p's c[m] = A[m][p], m >= p), its diagonal replaced by diag where REPLACE, -> packed
+// s.L, the other entries of s.L zeroed
+template <bool REPLACE>
+__device__ __forceinline__ void pack_L(Sim& s, const float (&c)[PP], float diag, int pd, int lane_) {
+  const int lane = opaque_lane(lane_);
+  for (int e = lane; e < NTRI + 2; e += WL) s.L[e] = 0.f;
+  static_for<0, PP, 1>([&](auto mc) {
+    constexpr int m = decltype(mc)::value;
+    const float at = lane_sel<PathEntry<m>::m>(__int_as_float(path_packed<m>(pd, lane)), __int_as_float(LSINK + lane));
+    s.L[__float_as_int(at)] = REPLACE ? lane_sel<PathEq<m>::m>(diag, c[m]) : c[m];
+  });
+  wsync();
+}
+// and back: the rows and columns without a dof 0
+__device__ __forceinline__ void unpack_L(const Sim& s, float (&c)[PP], int pd, int lane_) {
+  const int lane = opaque_lane(lane_);
+  static_for<0, PP, 1>([&](auto mc) {
+    constexpr int m = decltype(mc)::value;
+    const float x = s.L[m < 12 || lane >= 32 ? path_packed<m>(pd, lane) : 0];
+    c[m] = m < 12 ? lane_sel0<PATH_VALID>(x) : lane_sel0<PATH_ARMS>(x);
+  });
+  wsync();
+}
+
+// A value on the dof lanes' LDS vector x, on every lane of the path layout (0 on the lanes without a dof)
+__device__ __forceinline__ float path_value(const float* x, int pd) { return lane_sel0<PATH_VALID>(x[pd]); }
+__device__ __forceinline__ float dof_value(float x, int lane) {  // and back: a path-layout value on the dof lanes
+  return lane_of(x, owner_lane(min(lane, NV - 1)));
 }
 
 // ============================================================================================== smooth dynamics
@@ -76,26 +115,21 @@ __device__ __forceinline__ void apply_inertia(const float* J, const float* w, co
   for (int k = 0; k < 3; k++) f[k] = J[9] * v[k] - hw[k];
 }
 
-// the packed lower triangle of M + dg diag(kv) into s.L for the factorization: zeros, then each dof lane's chain
-// entries (M has the tree's sparsity: its nonzeros in row i are on the chain of dof i's body)
-__device__ __forceinline__ void m_to_L(Sim& s, int lane, float dg) {
-  for (int e = lane; e < NTRI + 2; e += WL) s.L[e] = 0.f;
-  if (lane < NV) {
-    const int bi = lane < 6 ? 1 : lane - 4;
-    unsigned ch[4];
-    for (int k = 0; k < 4; k++) ch[k] = s.chain[bi][k];
-    float* row = s.L + tri(lane, 0);
-#pragma unroll
-    for (int t = 0; t < MAXCHAIN; t++) {
-      const int j = chain_dof_row(ch, t, lane);
-      row[j] = s.M[lane][j];
-    }
-    row[lane] = s.M[lane][lane] + dg * cKv[lane];  // after the entries (same wave, program order)
-  }
-  wsync();
+// (M + dg diag(kv))^-1 b on the dof lanes, b an LDS vector over the dofs (36 words); the factor's rows are left in c
+// (and s.pf), its diagonal in *diag
+__device__ __forceinline__ float solve_M(Sim& s, float dg, const float* b, int pd, int lane, float (&c)[PP], float* diag) {
+  const PathRow row = path_row(s.M[pd], s.M[NV], lane);
+  const float dv = lane_sel0<PATH_VALID>(s.M[pd][pd] + dg * cKv[min(pd, NV - 1)]);
+  static_for<0, PP, 1>([&](auto mc) {
+    constexpr int m = decltype(mc)::value;
+    c[m] = path_entry<m>(row);
+    if (dg != 0.f) c[m] = lane_sel<PathEq<m>::m>(dv, c[m]);
+  });
+  *diag = path_factor(c, s.pf, lane);
+  return dof_value(path_solve(s.pf, c, *diag, path_value(b, pd), lane), lane);
 }
 
-__device__ void smooth(Sim& s, int lane) {
+__device__ void smooth(Sim& s, int pd, int lane) {
   // each hinge body's local transform, one lane per body: q_l = quat (x) hinge rotation, the body's offset in its
   // parent's frame p_b, and the hinge axis in the parent's frame a_l = quat a (the hinge rotation keeps its own axis)
   if (lane >= 2 && lane < NB) {
@@ -230,7 +264,7 @@ __device__ void smooth(Sim& s, int lane) {
   }
   wsync();
   // bias forces (qfrc_bias) projected on the dofs, CRBA row of dof `lane`, actuators
-  for (int e = lane; e < NV * MSTRIDE; e += WL) (&s.M[0][0])[e] = 0.f;
+  for (int e = lane; e < (NV + 1) * MSTRIDE; e += WL) (&s.M[0][0])[e] = 0.f;
   float bias = 0.f;
   if (lane < NV) {
     const int bi = lane < 6 ? 1 : lane - 4;
@@ -276,9 +310,8 @@ __device__ void smooth(Sim& s, int lane) {
   wsync();
   PROF(PH_SCRBA);
   // qacc_smooth = M^-1 qfrc_smooth
-  m_to_L(s, lane, 0.f);
-  factor_L(s, lane);
-  float x = ltl_solve(s.L, lane < NV ? s.qsm[lane] : 0.f, lane);
+  float c[PP], diag;
+  const float x = solve_M(s, 0.f, s.qsm, pd, lane, c, &diag);
   if (lane < NV) s.qacc0[lane] = x;
   wsync();
 }
@@ -450,7 +483,8 @@ __device__ __forceinline__ float matvec(const Sim& s, const float* v, int lane_)
 }
 
 // ============================================================================================== Newton
-struct NewtonOut { int it; bool conv, fresh; };  // fresh: s.L holds H's factor at the final zones
+// fresh: the factor is H's at the final zones; pattern, diag: where it is (0: s.pf and diag, else s.L)
+struct NewtonOut { int it, pattern; float diag; bool conv, fresh; };
 
 // The floor contacts are the contact lanes [0, nf) sorted by body (the floor pairs come first in pair order, sorted by
 // body, and contacts are compacted in pair order), and the bodies a dof moves are one run of body ids
@@ -588,8 +622,9 @@ __device__ __forceinline__ void contact_stiffness(const Rows& R, const float* dd
   K[15] = Kf[0][0]; K[16] = Kf[1][1]; K[17] = Kf[2][2]; K[18] = Kf[0][1]; K[19] = Kf[0][2]; K[20] = Kf[1][2];
 }
 
-// H = M + J' D J on the rows with x < 0, packed into s.L (lane i writes row i); returns the factorization pattern its
-// contacts between robot bodies need (factor_L: 0 the tree's sparsity, 1 the common self-contact fill, 2 dense).
+// H = M + J' D J on the rows with x < 0; returns the factorization its contacts between robot bodies need: 0 the
+// tree's sparsity, H's lower triangle in the path layout in c (path_factor); else H packed in s.L (factor_L: 1 the
+// common self-contact fill, 2 dense).
 //   Floor contacts: J'CJ of a contact on body B is S_i' K S_j on every pair of dofs moving B, with K = Phi' C Phi its
 //   6x6 stiffness about O. Dof i takes the sum of K over the floor contacts on the bodies it moves, one lane run
 //   (floor_run) read from the prefix sums of K over the lanes, accumulates (n, f) = (that sum) S_i, and
@@ -597,10 +632,7 @@ __device__ __forceinline__ void contact_stiffness(const Rows& R, const float* dd
 //   Contacts between two robot bodies: J'CJ = sum over the active pyramid edges t of u_t u_t', u_t = sqrt(D) J' e_t,
 //   u_t[d] = sigma_d S_d . (r x e_t, e_t) with sigma_d = (dof d moves body 2) - (dof d moves body 1); added as
 //   U U' on the matrix cores (fp32 MFMA), SELF_BATCH contacts (4 edges each) a batch.
-//   clear: zero s.L first. Not needed when s.L holds a factor with the tree's sparsity (of M or of an earlier H
-//   without contacts between robot bodies): such a factor is exactly 0 off the pattern, and the rows below overwrite
-//   every entry on it.
-__device__ __forceinline__ int hessian(Sim& s, const Rows& R, int lane, bool con, bool clear) {
+__device__ __forceinline__ int hessian(Sim& s, const Rows& R, int pd, int lane, bool con, float (&c)[PP]) {
   float d[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) d[t] = (con && t < R.nr && R.jar[t] < 0.f) ? R.D : 0.f;
@@ -630,33 +662,28 @@ __device__ __forceinline__ int hessian(Sim& s, const Rows& R, int lane, bool con
     f[2] = k[8] * w[0] + k[11] * w[1] + k[14] * w[2] + k[19] * v[0] + k[20] * v[1] + k[17] * v[2];
   }
   PROF(PH_HCOMP);
-  // rows of H: zero, then M[i][j] + S_j . (n, f) on the ancestor dofs j of i (M's nonzeros are on these chains)
-  if (clear)
-    for (int e = lane; e < NTRI + 2; e += WL) s.L[e] = 0.f;
-  if (lane < NV) {
-    const int bi = lane < 6 ? 1 : lane - 4;
-    // the chain of dof i's body: its ancestor dofs (and the root's j <= i). Every load first (S rows, M entries:
-    // independent of the stores into L), then the stores of the chain's entries
-    unsigned ch[4];
-    for (int k = 0; k < 4; k++) ch[k] = s.chain[bi][k];
-    float* row = s.L + tri(lane, 0);
+  // H[m][p] = M[m][p] + S_p . (n, f)_m down the path, every (n, f) moved from its dof's lane to the path layout (lane
+  // NV's are 0)
+  {
+    const PathRow row = path_row(s.M[pd], s.M[NV], lane);
+    float mc[PP], pn[3], pf[3];
+    static_for<0, PP, 1>([&](auto ec) { mc[decltype(ec)::value] = path_entry<decltype(ec)::value>(row); });
 #pragma unroll
-    for (int t0 = 0; t0 < MAXCHAIN; t0 += 8) {  // 8 entries a batch
-      float hv[8];
-      int hj[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const int j = chain_dof_row(ch, t0 + e, lane);
-        hj[e] = j;
-        hv[e] = s.M[lane][j] + (s.S[j][0] * n[0] + s.S[j][1] * n[1] + s.S[j][2] * n[2] + s.S[j][4] * f[0]
-                                + s.S[j][5] * f[1] + s.S[j][6] * f[2]);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; e++) row[hj[e]] = hv[e];  // the clamped entries store the diagonal's value again
+    for (int e = 0; e < 3; e++) { pn[e] = lane_of(n[e], pd); pf[e] = lane_of(f[e], pd); }
+    const float pw[3] = {s.S[pd][0], s.S[pd][1], s.S[pd][2]}, pv[3] = {s.S[pd][4], s.S[pd][5], s.S[pd][6]};
+    path_products(c, mc, pw, pv, pn, pf);
+    const float lim = R.lsg != 0.f && R.ljar < 0.f ? R.lD : 0.f;  // the limit rows in their zone, on the diagonal
+    if (ballot(lim != 0.f)) {
+      const float pl = lane_of(lim, pd);
+      static_for<0, PP, 1>([&](auto ec) {
+        constexpr int m = decltype(ec)::value;
+        c[m] = lane_sel<PathEq<m>::m>(c[m] + pl, c[m]);
+      });
     }
-    if (R.lsg != 0.f && R.ljar < 0.f) s.L[tri(lane, lane)] += R.lD;
   }
   PROF(PH_HROWS);
+  if (selfm == 0ull) return 0;
+  pack_L<false>(s, c, 0.f, pd, lane);
   for (unsigned long long m = selfm; m;) {  // contacts between two robot bodies, SELF_BATCH a batch
     unsigned long long bm = 0ull;
     for (int q = 0; q < SELF_BATCH && m; q++) { bm |= m & (~m + 1ull); m &= m - 1ull; }
@@ -761,11 +788,13 @@ __device__ __forceinline__ int hessian(Sim& s, const Rows& R, int lane, bool con
     cls = anc ? 0 : common ? 1 : 2;
   }
   const unsigned all = wor((unsigned)cls);
-  return all == 0u ? 0 : (all & 2u) ? 2 : 1;
+  if (all != 0u) return (all & 2u) ? 2 : 1;
+  unpack_L(s, c, pd, lane);
+  return 0;
 }
 
 
-__device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int lane, bool con, int iterations) {
+__device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int pd, int lane, bool con, int iterations) {
   // warm start against qacc_smooth: keep the cheaper (step.py:1974-1988)
   refresh(s, R, lane, con);
   float cost = wsum(lane_cost(s, R, lane));
@@ -784,24 +813,26 @@ __device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int lane, bool con,
     cost = cost0;
   }
   newton_grad(s, R, lane, con);
-  int it = 0, lpat = 0;  // lpat: the pattern of the factor in s.L (the smooth dynamics leave M's, the tree's)
+  int it = 0, pattern = 0;  // pattern: where H's factor is (0: s.pf and diag, else s.L)
+  float diag = 1.f;
   bool conv = false, zsame = false;
   while (it < iterations) {
     // a compiler barrier: LDS values are loaded where they are used inside the iteration, not hoisted out of the loop
     // into registers held across all of it
     asm volatile("" ::: "memory");
-    float p;
+    float p, c[PP];
     PROF(PH_NINIT);
-    if (zsame) {  // no row changed its zone in the last step: H, and so its factor in s.L, are unchanged
-      p = ltl_solve(s.L, lane < NV ? -s.grad[lane] : 0.f, lane);
-    } else {
-      const int pattern = hessian(s, R, lane, con, lpat != 0);
+    if (!zsame) {  // else no row changed its zone in the last step: H, and so its factor, are unchanged
+      pattern = hessian(s, R, pd, lane, con, c);
       PROF(PH_HESS);
-      factor_L(s, lane, pattern);
-      lpat = pattern;
+      if (pattern == 0) diag = path_factor(c, s.pf, lane);
+      else factor_L(s, lane, pattern);
       PROF(PH_FACTOR);
-      p = ltl_solve(s.L, lane < NV ? -s.grad[lane] : 0.f, lane);
+    } else if (pattern == 0) {
+      path_load(s.pf, c, lane);
     }
+    if (pattern == 0) p = dof_value(path_solve(s.pf, c, diag, -path_value(s.grad, pd), lane), lane);
+    else p = ltl_solve(s.L, lane < NV ? -s.grad[lane] : 0.f, lane);
     PROF(PH_SOLVE);
 #ifdef G1_PROFILE
     if (lane == 0) s.prof_acc[PH_ITERS] += 1;
@@ -904,7 +935,7 @@ __device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int lane, bool con,
     conv = improvement < kTol || kScale * gn < kTol;
     if (conv) break;
   }
-  return NewtonOut{it, conv, it > 0 && zsame};
+  return NewtonOut{it, pattern, diag, conv, it > 0 && zsame};
 }
 
 // ============================================================================================== one substep
@@ -926,7 +957,8 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
     tape_put(rec + REC_QVEL, s.qvel, NV, REC_ASTAR - REC_QVEL, lane);
   }
   PROF(PH_TAPE);
-  smooth(s, lane);
+  const int pd = path_lane_dof(lane);  // this lane's dof in the path layout (NV: none)
+  smooth(s, pd, lane);
   PROF(PH_SMOOTH);
   collision(s, lane);
   PROF(PH_COLLIDE);
@@ -1026,14 +1058,20 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
     }
     sing = ballot(nu < SINGULAR_NU) != 0ull;
   }
-  const NewtonOut no = newton(s, R, lane, con, iterations);
+  NewtonOut no = newton(s, R, pd, lane, con, iterations);
   PROF(PH_NINIT);
   if (lane == 0) s.niter = no.it;
   if (rec) {  // the final zones, and H's factor at them (assembled again when the last step changed a zone)
+    float c[PP];
     if (!no.fresh) {
-      const int pattern = hessian(s, R, lane, con, true);
-      factor_L(s, lane, pattern);
+      no.pattern = hessian(s, R, pd, lane, con, c);
+      if (no.pattern == 0) no.diag = path_factor(c, s.pf, lane);
+      else factor_L(s, lane, no.pattern);
+    } else if (no.pattern == 0) {
+      path_load(s.pf, c, lane);
+      wsync();
     }
+    if (no.pattern == 0) pack_L<true>(s, c, no.diag, pd, lane);
     tape_put(rec + REC_LH, s.L, NTRI, REC_LQ - REC_LH, lane);
     unsigned cz = 0u;
     for (int t = 0; t < 4; t++) cz |= (t < R.nr && R.jar[t] < 0.f) ? 1u << t : 0u;
@@ -1069,11 +1107,11 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
   PROF(PH_TAPE);
   // implicitfast: (M + h kv) a_adv = M a*
   {
-    m_to_L(s, lane, kH);
-    factor_L(s, lane);
-    const float adv = ltl_solve(s.L, lane < NV ? s.Ma[lane] : 0.f, lane);
+    float c[PP], diag;
+    const float adv = solve_M(s, kH, s.Ma, pd, lane, c, &diag);
     if (lane < NV) s.qvel[lane] += kH * adv;
     if (rec) {
+      pack_L<true>(s, c, diag, pd, lane);
       // L_Q, its off-pattern positions carrying the body frames FK left at the substep's start (g1_tape.h): they
       // are written into the factor's zeros in LDS first (s.L is factored afresh before its next use); a position's
       // fourth word, which nothing writes in s.X, as 0
@@ -1155,6 +1193,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   if (lane < 3) s.com[lane] = ic;
   if (lane == 0) { s.fric = ifr; s.flags = 0; s.niter = 0; s.dcnt = 0; s.acost = 0; }
   s.dsub[lane] = lane < NV ? cTree.dofmask32[lane] : 0u;
+  if (lane < 8) s.S[NV][lane] = 0.f;
   chain_table(s.chain, lane);
 #ifdef G1_PROFILE
   if (lane < NPHASE) s.prof_acc[lane] = 0;

@@ -1,0 +1,76 @@
+"""The factorizations and solves in the path layout (csrc/g1_path.h) at the places where it can go wrong: no
+constraint rows at all; a limit row on every hinge (every diagonal entry), on the waist's three (shared by both arm
+paths), on one leg's or one arm's; contacts on one limb; contacts between robot bodies, whose assembly goes through
+the packed form, on and off one path. One substep, from its tape record against float64 (the oracle)."""
+import numpy as np
+import pytest
+
+import oracle
+from nablaengine_amd import synthetic
+
+pytestmark = pytest.mark.gpu
+KEYS = ("qpos", "qvel", "warm", "ctrl", "friction", "com")
+REC_FLAGS, REC_ASTAR, REC_AADV, REC_LH, REC_LQ = 1, 128, 164, 200, 832
+HINGES = {"legs_left": (6, 12), "legs_right": (12, 18), "waist": (18, 21), "arm_left": (21, 28), "arm_right": (28, 35),
+          "all": (6, 35)}
+
+
+def _states(kind, n):
+    st = synthetic.states(n, config=4 if kind == "tangled" else 1, seed=77)
+    rng = np.random.default_rng(78)
+    if kind == "tangled":
+        return st
+    st["qpos"][:, 2] = 2.0  # in the air
+    if kind in HINGES:  # past the upper limit of each hinge of the range
+        hi = np.asarray(synthetic.model()["dof_range"]).reshape(35, 2)[:, 1]
+        a, b = HINGES[kind]
+        st["qpos"][:, a + 1:b + 1] = hi[a:b] + rng.uniform(0.01, 0.05, (n, b - a))
+    elif kind == "one_foot":  # rolled about x until only one foot's spheres touch
+        st["qpos"][:, 2] = 0.74
+        st["qpos"][:, 3:7] = [np.cos(0.15), np.sin(0.15), 0, 0]
+    return {k: np.ascontiguousarray(v, np.float32) for k, v in st.items()}
+
+
+def _unpack(x):
+    L = np.zeros((35, 35))
+    L[np.tril_indices(35)] = x[:630]
+    return L
+
+
+@pytest.mark.parametrize("kind", ["flight", "all", "waist", "legs_left", "legs_right", "arm_left", "arm_right",
+                                  "one_foot", "tangled"])
+def test_path_factors_vs_oracle(kind):
+    """L_Q against float64's factor of M + h kv, L_H' L_H against H at the final zones, and a_adv's residual in
+    (M + h kv) a_adv = M a*. Tolerances: the elimination's backward error is at most about n eps = 35 x 6e-8 = 2e-6 of
+    the largest entry, and M and H themselves are sums of some tens of float32 terms (a few 1e-7 each): 1e-5; the
+    residual is that of the factor times |x| (1e-5 |Q| |a_adv|, rows against the largest)."""
+    import torch
+    from nablaengine_amd import torch_ffi
+    B = 12
+    st = _states(kind, B)
+    args = [torch.from_numpy(st[k]).cuda() for k in KEYS]
+    _, _, _, info, tape = torch_ffi.forward(*args, iterations=50, substeps=1, tape=True)
+    tape, info = tape.cpu().numpy(), info.cpu().numpy()
+    m = synthetic.model()
+    hkv = m["timestep"] * np.diag(np.asarray(m["dof_kv"]))
+    tree = np.array([[bool((m["body_ancmask"][m["dof_body"][i]] >> m["dof_body"][j]) & 1) for j in range(35)]
+                     for i in range(35)])
+    checked = 0
+    for w in range(B):
+        s = {k: st[k][w].astype(np.float64) for k in KEYS}
+        M, H = oracle.substep_hessian(s["qpos"], s["qvel"], s["warm"], s["ctrl"], float(s["friction"]), s["com"])
+        rec = tape[w]
+        ref = oracle.ltl(M + hkv)
+        assert np.abs(_unpack(rec[REC_LQ:]) * tree - ref).max() <= 1e-5 * np.abs(ref).max(), w
+        a, adv = rec[REC_ASTAR:REC_ASTAR + 35].astype(np.float64), rec[REC_AADV:REC_AADV + 35].astype(np.float64)
+        res = (M + hkv) @ adv - M @ a
+        assert np.abs(res).max() <= 1e-5 * (np.abs(M + hkv) @ np.abs(adv)).max(), w
+        if not rec[REC_FLAGS:REC_FLAGS + 1].view(np.uint32)[0] & (4 | 16 | (1 << 9)):
+            L = _unpack(rec[REC_LH:])
+            checked += np.abs(L.T @ L - H).max() <= 1e-5 * np.abs(H).max()
+    assert checked >= B - 2, checked  # a world whose float32 and float64 solves end in different zones differs by a row
+    if kind in HINGES:
+        a, b = HINGES[kind]
+        assert (info[:, 2] >= b - a).all(), info  # the limit rows are there
+    if kind == "flight":
+        assert (info[:, 2] == 0).sum() >= 4, info  # worlds without any row (a hand may touch the hip in the others)
