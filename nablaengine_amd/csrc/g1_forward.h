@@ -9,6 +9,9 @@ constexpr int MSTRIDE = 36;
 // the smooth dynamics' per-body row: force, moment about O, spatial inertia (10 of 12), each 16-byte aligned
 constexpr int SM_F = 0, SM_T = 4, SM_I = 8, SMW = 20;
 
+constexpr int SELF_BATCH = 4;   // contacts between two robot bodies per outer-product batch (4 edge rows each)
+constexpr int SELF_CHUNK = 16;  // and those whose edge rows are formed at once
+
 struct __align__(16) Sim {
   // the dof vectors padded to 36 entries (16-byte multiples; matvec reads them as float4s)
   float qpos[40], qvel[36], qacc[36], ctrl[32], com[4];
@@ -38,9 +41,7 @@ struct __align__(16) Sim {
     struct { float gx[NGEOM][4], gq[NGEOM][4]; float stage[MAXCON][16]; unsigned short cand[NPAIR + 2]; } col;
     struct {
       float bw[NB][8];  // body spatial velocity of a dof vector: angular (0..2), velocity of O (4..6)
-      struct { float psi[16][8]; float U[48][17]; } h;  // Hessian: a batch of self-contact rows (<= 16);
-                                                         // U's rows past the dofs zero (MFMA tiles of 16); rows
-                                                         // padded to 17 floats: no LDS bank conflicts down a column
+      float psi[4 * SELF_CHUNK][8];  // Hessian: the edge rows of a chunk of contacts between robot bodies
     } nt;
   } u;
 };

@@ -378,15 +378,22 @@ __device__ void collision(Sim& s, int lane) {
 // ============================================================================================== rows
 // impedance (k, b, imp) of a row at distance pos, solref / solimp with refsafe (step.py:1157-1171 kbimp); the model's
 // solimp power is 2
-__device__ __forceinline__ void kbimp(const float* solref, const float* solimp, float pos, float* k, float* b,
-                                      float* imp) {
-  float tc = fmaxf(solref[0], 2.f * kH), dr = solref[1];
-  float dmin = fminf(fmaxf(solimp[0], 1e-4f), 0.9999f), dmax = fminf(fmaxf(solimp[1], 1e-4f), 0.9999f);
-  float width = fmaxf(1e-15f, solimp[2]), mid = fminf(fmaxf(solimp[3], 1e-4f), 0.9999f);
-  *k = 1.f / fmaxf(1e-15f, dmax * dmax * tc * tc * dr * dr);
-  *b = 2.f / fmaxf(1e-15f, dmax * tc);
+// (solref and solimp as compile-time values: read from constant memory, what depends on them alone was computed once a
+// world and held in 17 registers through every substep, or spilled)
+constexpr Arr<float, 2> JSOLREF = to_float(JNT_SOLREF), PSOLREF = to_float(PAIR_SOLREF);
+constexpr Arr<float, 5> JSOLIMP = to_float(JNT_SOLIMP), PSOLIMP = to_float(PAIR_SOLIMP);
+static_assert(JNT_SOLIMP[4] == 2.0 && PAIR_SOLIMP[4] == 2.0, "kbimp assumes the solimp power 2");
+constexpr float cmax(float a, float b) { return a < b ? b : a; }
+constexpr float cclamp(float x, float lo, float hi) { return x < lo ? lo : x > hi ? hi : x; }
+template <const Arr<float, 2>& SOLREF, const Arr<float, 5>& SOLIMP>
+__device__ __forceinline__ void kbimp(float pos, float* k, float* b, float* imp) {
+  constexpr float tc = cmax(SOLREF.v[0], 2.f * kH), dr = SOLREF.v[1];
+  constexpr float dmin = cclamp(SOLIMP.v[0], 1e-4f, 0.9999f), dmax = cclamp(SOLIMP.v[1], 1e-4f, 0.9999f);
+  constexpr float width = cmax(1e-15f, SOLIMP.v[2]), mid = cclamp(SOLIMP.v[3], 1e-4f, 0.9999f);
+  *k = 1.f / cmax(1e-15f, dmax * dmax * tc * tc * dr * dr);
+  *b = 2.f / cmax(1e-15f, dmax * tc);
   float x = fabsf(pos) / width;
-  if (dmin == dmax || solimp[2] <= 1e-15f) *imp = 0.5f * (dmin + dmax);
+  if (dmin == dmax || SOLIMP.v[2] <= 1e-15f) *imp = 0.5f * (dmin + dmax);
   else if (x <= 0.f) *imp = dmin;
   else if (x >= 1.f) *imp = dmax;
   else {
@@ -394,12 +401,6 @@ __device__ __forceinline__ void kbimp(const float* solref, const float* solimp, 
     *imp = fminf(fmaxf(dmin + y * (dmax - dmin), dmin), dmax);
   }
 }
-
-__constant__ inline Arr<float, 2> cJSolref = to_float(JNT_SOLREF);
-__constant__ inline Arr<float, 5> cJSolimp = to_float(JNT_SOLIMP);
-__constant__ inline Arr<float, 2> cPSolref = to_float(PAIR_SOLREF);
-__constant__ inline Arr<float, 5> cPSolimp = to_float(PAIR_SOLIMP);
-static_assert(JNT_SOLIMP[4] == 2.0 && PAIR_SOLIMP[4] == 2.0, "kbimp assumes the solimp power 2");
 
 // body spatial velocities of the dof vector v (LDS): bw[b] = sum over b's chain of S_d v_d, down the tree: the root
 // body's from the root's 6 dofs (S_0..2 = (0; e_k), S_3..5 = (w_k; 0): v[0..2] and 3 columns), then each hinge body's
@@ -414,8 +415,8 @@ __device__ __forceinline__ void body_vel(Sim& s, const float* v, int lane) {
   const int so = comp ? (c < 3 ? c : c + 1) : 0;  // the component's place in a row of S and bw: w 0..2, v 4..6
   const int lo = g == 0 ? PATHS.lo[0] : g == 1 ? PATHS.lo[1] : g == 2 ? PATHS.lo[2] : PATHS.lo[3];
   const int hi = g == 0 ? PATHS.hi[0] : g == 1 ? PATHS.hi[1] : g == 2 ? PATHS.hi[2] : PATHS.hi[3];
-  float* sink = &s.u.nt.h.psi[0][0] + (lane & 7);  // 8 * PATH_STEPS + 7 floats: inside psi
-  static_assert(8 * PATH_STEPS + 8 <= 16 * 8, "the sink inside psi");
+  float* sink = &s.u.nt.psi[0][0] + (lane & 7);  // 8 * PATH_STEPS + 7 floats: inside psi
+  static_assert(8 * PATH_STEPS + 8 <= 4 * SELF_CHUNK * 8, "the sink inside psi");
   const float rw = s.S[3][so] * v[3] + s.S[4][so] * v[4] + s.S[5][so] * v[5];
   float T = c < 3 ? rw : v[comp ? c - 3 : 0];
   (comp && g < 2 ? &s.u.nt.bw[1 - g][so] : sink)[0] = g == 0 ? T : 0.f;  // the root body; the world body 0
@@ -587,7 +588,6 @@ __device__ void refresh(Sim& s, Rows& R, int lane, bool con, bool smooth = false
   R.ljar = ljv - R.laref;
 }
 
-constexpr int SELF_BATCH = 4;  // contacts between two robot bodies per outer-product batch (4 edge rows each)
 
 // a floor contact's 6x6 stiffness K = Phi' C Phi about O (21 floats: Kaa 6, Kal 9, Kf 6), C from the curvatures d of
 // its pyramid rows in the frame basis; zero where !on
@@ -622,6 +622,120 @@ __device__ __forceinline__ void contact_stiffness(const Rows& R, const float* dd
   K[15] = Kf[0][0]; K[16] = Kf[1][1]; K[17] = Kf[2][2]; K[18] = Kf[0][1]; K[19] = Kf[0][2]; K[20] = Kf[1][2];
 }
 
+// s.L += the contacts between robot bodies selfm (lanes), sum over the active pyramid edges t of u_t u_t' with u_t =
+// sqrt(D) J' e_t, u_t[i] = sigma_i S_i . (r x e_t, e_t), sigma_i = (dof i moves body 2) - (dof i moves body 1). On the
+// matrix cores (v_mfma_f32_16x16x4f32: lane l gives A[l % 16][l / 16] and B[l / 16][l % 16], holds C[4 (l / 16) + e]
+// [l % 16]), a batch of SELF_BATCH contacts at a time, its 16 edge vectors psi = (r x e_t, e_t) in LDS with row
+// 4 t + q for edge t of contact q. C' = Psi S' (16 x 8 x 48: S's two unused slots and the rows past the dofs zero) then
+// leaves contact e's edge l / 16 on dof 16 k + l % 16 in C'[k][e]: with its sign that is already the operand of
+// contact e's step of U U' (k = its 4 edges), both as A and as B, with no pass through LDS. The products are summed
+// over a batch from 0 and the sums added to H's lower 16 x 16 tiles, which stay in registers over all batches (dofs
+// 32..34 are 3 rows of the last tile row: rows e < 3 of lanes 0..15). The psi of up to SELF_CHUNK contacts are formed
+// at once, each on its contact's lane. Bound by latency: with U passed through LDS, every
+// tile entry loaded, added to and stored per batch, and each batch's psi formed by itself, a Hessian with such contacts
+// took 10.9 k cycles in the heaviest 1% of 512 standing worlds, now 5.7 k (forward + VJP of 512 worlds 628 -> 522 us,
+// of 4096 contact-heavy ones 982 -> 946 us).
+__device__ __forceinline__ void add_self_contacts(Sim& s, const Rows& R, const float* d, unsigned long long selfm,
+                                                  int lane_) {
+  const int lane = opaque_lane(lane_), lr = lane & 15, lk = lane >> 4;
+  float sk[3][2];  // S of dof 16 t + lr, slots lk and 4 + lk
+  unsigned dm[3];  // the bodies it moves
+#pragma unroll
+  for (int t = 0; t < 3; t++) {
+    const int i = min(16 * t + lr, NV);  // row NV is 0
+    dm[t] = s.dsub[16 * t + lr];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const float x = s.S[i][4 * h + lk];
+      sk[t][h] = lk == 3 ? 0.f : x;
+    }
+  }
+  // H's tiles: entry (16 ti + 4 lk + e, 16 tj + lr); the lanes off the triangle use their sink. (The addresses are
+  // formed anew for the store: held across the batches they would cost 12 registers.)
+  float H[3][3][4];
+  auto tiles = [&](auto f) {
+    const int ln = opaque_lane(lane), r = ln & 15, k = ln >> 4;
+    float* const sink = s.L + LSINK + ln;
+    static_for<0, 3, 1>([&](auto ic) {
+      static_for<0, 4, 1>([&](auto ec) {
+        constexpr int ti = decltype(ic)::value, e = decltype(ec)::value;
+        if constexpr (16 * ti + e < NV) {
+          float* const row = s.L + tri(16 * ti + 4 * k + e, 0) + r;
+          static_for<0, ti + 1, 1>([&](auto jc) {
+            constexpr int tj = decltype(jc)::value;
+            const bool in = (ti < 2 || k == 0) && (ti != tj || r <= 4 * k + e);
+            f(ic, jc, ec, in ? row + 16 * tj : sink);
+          });
+        }
+      });
+    });
+  };
+  tiles([&](auto ic, auto jc, auto ec, float* p) { H[decltype(ic)::value][decltype(jc)::value][decltype(ec)::value] = *p; });
+  for (unsigned long long m = selfm; m;) {
+    const int q = prefix_count(m, lane);
+    if (((m >> lane) & 1ull) && q < SELF_CHUNK) {  // this contact's 4 edge rows: sqrt(D) (r x e_t, e_t), e_t = n +- mu t1, n +- mu t2
+      const float sd = sqrtf(R.D);
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        float e[3];
+        const float sg = (t & 1) ? -R.mu : R.mu;
+        const float* ta = R.fr + 3 * (1 + (t >> 1));
+        for (int k = 0; k < 3; k++) e[k] = R.dim == 3 ? R.fr[k] + sg * ta[k] : (t == 0 ? R.fr[k] : 0.f);
+        const float sc = d[t] != 0.f ? sd : 0.f;
+        float re[3];
+        cross(R.r, e, re);
+        float4* o = reinterpret_cast<float4*>(s.u.nt.psi[16 * (q >> 2) + 4 * t + (q & 3)]);
+        o[0] = make_float4(sc * re[0], sc * re[1], sc * re[2], 0.f);
+        o[1] = make_float4(sc * e[0], sc * e[1], sc * e[2], 0.f);
+      }
+    }
+    wsync();
+#pragma unroll 1
+    for (int b = 0; b < SELF_CHUNK / SELF_BATCH && m; b++) {
+      const float* pr = s.u.nt.psi[16 * b + lr] + lk;
+      const float p0 = pr[0], p1 = pr[4];
+      mfma4 u[3];
+#pragma unroll
+      for (int t = 0; t < 3; t++) {
+        u[t] = mfma4{0.f, 0.f, 0.f, 0.f};
+        u[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0, sk[t][0], u[t], 0, 0, 0);
+        u[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1, sk[t][1], u[t], 0, 0, 0);
+      }
+      mfma4 acc[3][3];
+#pragma unroll
+      for (int ti = 0; ti < 3; ti++)
+#pragma unroll
+        for (int tj = 0; tj <= ti; tj++) acc[ti][tj] = mfma4{0.f, 0.f, 0.f, 0.f};
+      static_for<0, SELF_BATCH, 1>([&](auto ec) {
+        constexpr int e = decltype(ec)::value;
+        if (m) {
+          const int cl = __builtin_ctzll(m);
+          m &= m - 1ull;
+          const int b1 = rdli(R.b1, cl), b2 = rdli(R.b2, cl);
+          float op[3];
+#pragma unroll
+          for (int t = 0; t < 3; t++)
+            op[t] = (float)((int)((dm[t] >> b2) & 1u) - (int)((dm[t] >> b1) & 1u)) * u[t][e];
+#pragma unroll
+          for (int ti = 0; ti < 3; ti++)
+#pragma unroll
+            for (int tj = 0; tj <= ti; tj++)
+              acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[ti], op[tj], acc[ti][tj], 0, 0, 0);
+        }
+      });
+#pragma unroll
+      for (int ti = 0; ti < 3; ti++)
+#pragma unroll
+        for (int tj = 0; tj <= ti; tj++)
+#pragma unroll
+          for (int e = 0; e < (ti == 2 ? 3 : 4); e++) H[ti][tj][e] += acc[ti][tj][e];
+    }
+    wsync();
+  }
+  tiles([&](auto ic, auto jc, auto ec, float* p) { *p = H[decltype(ic)::value][decltype(jc)::value][decltype(ec)::value]; });
+  wsync();
+}
+
 // H = M + J' D J on the rows with x < 0; returns the factorization its contacts between robot bodies need: 0 the
 // tree's sparsity, H's lower triangle in the path layout in c (path_factor); else H packed in s.L (factor_L: 1 the
 // common self-contact fill, 2 dense).
@@ -629,9 +743,7 @@ __device__ __forceinline__ void contact_stiffness(const Rows& R, const float* dd
 //   6x6 stiffness about O. Dof i takes the sum of K over the floor contacts on the bodies it moves, one lane run
 //   (floor_run) read from the prefix sums of K over the lanes, accumulates (n, f) = (that sum) S_i, and
 //   H[i][j] = S_j . (n, f) on i's ancestor dofs j (the composite stiffness of i's subtree, as CRBA composites inertia).
-//   Contacts between two robot bodies: J'CJ = sum over the active pyramid edges t of u_t u_t', u_t = sqrt(D) J' e_t,
-//   u_t[d] = sigma_d S_d . (r x e_t, e_t) with sigma_d = (dof d moves body 2) - (dof d moves body 1); added as
-//   U U' on the matrix cores (fp32 MFMA), SELF_BATCH contacts (4 edges each) a batch.
+//   Contacts between two robot bodies: add_self_contacts.
 __device__ __forceinline__ int hessian(Sim& s, const Rows& R, int pd, int lane, bool con, float (&c)[PP]) {
   float d[4];
 #pragma unroll
@@ -684,98 +796,7 @@ __device__ __forceinline__ int hessian(Sim& s, const Rows& R, int pd, int lane, 
   PROF(PH_HROWS);
   if (selfm == 0ull) return 0;
   pack_L<false>(s, c, 0.f, pd, lane);
-  for (unsigned long long m = selfm; m;) {  // contacts between two robot bodies, SELF_BATCH a batch
-    unsigned long long bm = 0ull;
-    for (int q = 0; q < SELF_BATCH && m; q++) { bm |= m & (~m + 1ull); m &= m - 1ull; }
-    if (lane < 4 * SELF_BATCH)
-      for (int k = 0; k < 8; k++) s.u.nt.h.psi[lane][k] = 0.f;
-    if ((bm >> lane) & 1ull) {  // this contact's 4 edge rows: sqrt(D) (r x e_t, e_t), e_t = n +- mu t1, n +- mu t2
-      const int q = prefix_count(bm, lane);
-      const float sd = sqrtf(R.D);
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        float e[3];
-        const float sg = (t & 1) ? -R.mu : R.mu;
-        const float* ta = R.fr + 3 * (1 + (t >> 1));
-        for (int k = 0; k < 3; k++) e[k] = R.dim == 3 ? R.fr[k] + sg * ta[k] : (t == 0 ? R.fr[k] : 0.f);
-        const float sc = d[t] != 0.f ? sd : 0.f;
-        float re[3];
-        cross(R.r, e, re);
-        float* o = s.u.nt.h.psi[4 * q + t];
-        for (int k = 0; k < 3; k++) { o[k] = sc * re[k]; o[3 + k] = sc * e[k]; }
-        o[6] = __int_as_float(R.b1);
-        o[7] = __int_as_float(R.b2);
-      }
-    }
-    wsync();
-    {  // U[i][r] = sigma_r(i) S_i . psi_r (rows past the dofs zero): S Psi' (48 x 8 x 16, S's rows with its two
-       // unused slots 3 and 7 as zero columns) on the matrix cores, 3 row tiles x 2 k-steps, then the signs
-      const int ln = opaque_lane(lane);
-      const int lr = ln & 15, lk = ln >> 4;
-      const float* pr = s.u.nt.h.psi[lr];  // this lane's column r = lr
-      const int b1r = __float_as_int(pr[6]), b2r = __float_as_int(pr[7]);
-      float bv[2];
-#pragma unroll
-      for (int kk = 0; kk < 2; kk++) {
-        const int k = 4 * kk + lk;  // S's slot; psi's 0..5 are S's 0..2, 4..6
-        const float x = pr[k < 3 ? k : (k < 7 ? k - 1 : 0)];
-        bv[kk] = (k == 3 || k == 7) ? 0.f : x;
-      }
-#pragma unroll
-      for (int t = 0; t < 3; t++) {
-        const int ia = 16 * t + lr, ic = ia < NV ? ia : 0;
-        mfma4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 2; kk++) {
-          const int k = 4 * kk + lk;
-          const float x = s.S[ic][k];
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ia < NV && k != 3 && k != 7 ? x : 0.f, bv[kk], acc, 0, 0, 0);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int i = 16 * t + 4 * lk + e;
-          const unsigned di = s.dsub[i];  // 0 past the dofs
-          const float sg = (float)((int)((di >> b2r) & 1u) - (int)((di >> b1r) & 1u));
-          s.u.nt.h.U[i][lr] = sg * acc[e];
-        }
-      }
-    }
-    wsync();
-    {  // H += U U' on the matrix cores: 16 x 16 tiles (ti, tj <= ti) of the 48-row padding, k = the batch's edge rows
-      // in steps of 4 (v_mfma_f32_16x16x4f32: lane l gives A[l % 16][l / 16] and B[l / 16][l % 16], holds
-      // C[4 (l / 16) + e][l % 16]). Step kk takes U's columns 4 kk .. 4 kk + 3, contact kk's 4 edge rows, so a batch
-      // of nb contacts needs nb steps: the 6 tiles' chains are nb deep, not SELF_BATCH
-      const int lr = lane & 15, lk = lane >> 4;
-      const int nb = __popcll(bm);
-      mfma4 acc[6];
-#pragma unroll
-      for (int n = 0; n < 6; n++) acc[n] = mfma4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-      for (int kk = 0; kk < nb; kk++) {
-        float op[3];
-#pragma unroll
-        for (int t = 0; t < 3; t++) op[t] = s.u.nt.h.U[16 * t + lr][4 * kk + lk];
-        int n = 0;
-#pragma unroll
-        for (int ti = 0; ti < 3; ti++)
-#pragma unroll
-          for (int tj = 0; tj <= ti; tj++, n++)
-            acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[ti], op[tj], acc[n], 0, 0, 0);
-      }
-      int n = 0;
-#pragma unroll
-      for (int ti = 0; ti < 3; ti++)
-#pragma unroll
-        for (int tj = 0; tj <= ti; tj++, n++)
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const int i = 16 * ti + 4 * lk + e, j = 16 * tj + lr;
-            s.L[i < NV && j <= i ? tri(i, j) : LSINK + lane] += acc[n][e];  // off the triangle: the lane's sink
-          }
-    }
-    wsync();
-  }
-  wsync();
+  add_self_contacts(s, R, d, selfm, lane);
   // the factorization's pattern from the active contacts between robot bodies (body x < y): none when x is y's
   // ancestor (the coupling stays on y's chain); the common fill for a leg against the waist or its own arm, or the two
   // legs; else dense
@@ -1025,14 +1046,14 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
   if (con) contact_dots(s, R, vdot);
   if (R.lsg != 0.f) {
     float k, b, imp;
-    kbimp(cJSolref.v, cJSolimp.v, lpos, &k, &b, &imp);
+    kbimp<JSOLREF, JSOLIMP>(lpos, &k, &b, &imp);
     const float iw = cDinvw[lane];
     R.lD = 1.f / fmaxf(iw * (1.f - imp) / imp, 1e-15f);
     R.laref = -k * imp * lpos - b * (R.lsg * s.qvel[lane]);
   }
   if (con) {
     float k, b, imp;
-    kbimp(cPSolref.v, cPSolimp.v, dist, &k, &b, &imp);
+    kbimp<PSOLREF, PSOLIMP>(dist, &k, &b, &imp);
     float iw = piw;
     if (R.dim == 3) iw = (R.mu * R.mu * iw + iw) * 2.f * R.mu * R.mu / kImpratio;
     R.D = 1.f / fmaxf(iw * (1.f - imp) / imp, 1e-15f);

@@ -1,7 +1,7 @@
 """The factorizations and solves in the path layout (csrc/g1_path.h) at the places where it can go wrong: no
 constraint rows at all; a limit row on every hinge (every diagonal entry), on the waist's three (shared by both arm
 paths), on one leg's or one arm's; contacts on one limb; contacts between robot bodies, whose assembly goes through
-the packed form, on and off one path. One substep, from its tape record against float64 (the oracle)."""
+the packed form, on and off one path, fewer and more than are assembled at once. One substep, from its tape record against float64 (the oracle)."""
 import numpy as np
 import pytest
 
@@ -25,6 +25,10 @@ def _states(kind, n):
         hi = np.asarray(synthetic.model()["dof_range"]).reshape(35, 2)[:, 1]
         a, b = HINGES[kind]
         st["qpos"][:, a + 1:b + 1] = hi[a:b] + rng.uniform(0.01, 0.05, (n, b - a))
+    elif kind == "feet":  # the legs rolled inwards until the feet's 7 spheres each overlap: 1 to 28 contacts
+        st["qpos"][:, 7:19] = rng.normal(0.0, 0.03, (n, 12))
+        st["qpos"][:, 8] -= 0.16
+        st["qpos"][:, 14] += 0.16
     elif kind == "one_foot":  # rolled about x until only one foot's spheres touch
         st["qpos"][:, 2] = 0.74
         st["qpos"][:, 3:7] = [np.cos(0.15), np.sin(0.15), 0, 0]
@@ -38,7 +42,7 @@ def _unpack(x):
 
 
 @pytest.mark.parametrize("kind", ["flight", "all", "waist", "legs_left", "legs_right", "arm_left", "arm_right",
-                                  "one_foot", "tangled"])
+                                  "one_foot", "tangled", "feet"])
 def test_path_factors_vs_oracle(kind):
     """L_Q against float64's factor of M + h kv, L_H' L_H against H at the final zones, and a_adv's residual in
     (M + h kv) a_adv = M a*. Tolerances: the elimination's backward error is at most about n eps = 35 x 6e-8 = 2e-6 of
@@ -55,7 +59,7 @@ def test_path_factors_vs_oracle(kind):
     hkv = m["timestep"] * np.diag(np.asarray(m["dof_kv"]))
     tree = np.array([[bool((m["body_ancmask"][m["dof_body"][i]] >> m["dof_body"][j]) & 1) for j in range(35)]
                      for i in range(35)])
-    checked = 0
+    same = []
     for w in range(B):
         s = {k: st[k][w].astype(np.float64) for k in KEYS}
         M, H = oracle.substep_hessian(s["qpos"], s["qvel"], s["warm"], s["ctrl"], float(s["friction"]), s["com"])
@@ -67,10 +71,16 @@ def test_path_factors_vs_oracle(kind):
         assert np.abs(res).max() <= 1e-5 * (np.abs(M + hkv) @ np.abs(adv)).max(), w
         if not rec[REC_FLAGS:REC_FLAGS + 1].view(np.uint32)[0] & (4 | 16 | (1 << 9)):
             L = _unpack(rec[REC_LH:])
-            checked += np.abs(L.T @ L - H).max() <= 1e-5 * np.abs(H).max()
-    assert checked >= B - 2, checked  # a world whose float32 and float64 solves end in different zones differs by a row
+            if np.abs(L.T @ L - H).max() <= 1e-5 * np.abs(H).max():
+                same.append(w)
+    # a world whose float32 and float64 solves end in different zones differs by a row's D J J'; with two feet's worth of
+    # redundant contacts most do, so there it is enough that worlds past one chunk of edge rows are among the others
+    print(kind, "H agrees in", same, "contacts", info[:, 1].tolist())
+    assert len(same) >= (3 if kind == "feet" else B - 2), same
     if kind in HINGES:
         a, b = HINGES[kind]
         assert (info[:, 2] >= b - a).all(), info  # the limit rows are there
+    if kind == "feet":
+        assert info[same, 1].max() > 16 and (info[same, 1] % 4 != 0).any(), info
     if kind == "flight":
         assert (info[:, 2] == 0).sum() >= 4, info  # worlds without any row (a hand may touch the hip in the others)
