@@ -31,8 +31,8 @@ __device__ __forceinline__ void factor_L(Sim& s, int lane, int pattern) {
 #ifdef G1_PROFILE
   if (lane == 0) s.prof_acc[PH_DENSE] += 1;
 #endif
-  if (pattern == 1) ltl_factor<1>(s.L, lane);
-  else ltl_factor<2>(s.L, lane);
+  if (pattern == 1) ltl_factor<1>(s.u.nt.L, lane);
+  else ltl_factor<2>(s.u.nt.L, lane);
   wsync();
 }
 
@@ -48,15 +48,15 @@ __device__ __forceinline__ int path_packed(int pd, int lane) {
   return i * (i + 1) / 2 + pd;
 }
 // a lower triangle in the path layout (lane p's c[m] = A[m][p], m >= p), its diagonal replaced by diag where REPLACE, -> packed
-// s.L, the other entries of s.L zeroed
+// s.u.nt.L, the other entries of s.L zeroed
 template <bool REPLACE>
 __device__ __forceinline__ void pack_L(Sim& s, const float (&c)[PP], float diag, int pd, int lane_) {
   const int lane = opaque_lane(lane_);
-  for (int e = lane; e < NTRI + 2; e += WL) s.L[e] = 0.f;
+  for (int e = lane; e < NTRI + 2; e += WL) s.u.nt.L[e] = 0.f;
   static_for<0, PP, 1>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
     const float at = lane_sel<PathEntry<m>::m>(__int_as_float(path_packed<m>(pd, lane)), __int_as_float(LSINK + lane));
-    s.L[__float_as_int(at)] = REPLACE ? lane_sel<PathEq<m>::m>(diag, c[m]) : c[m];
+    s.u.nt.L[__float_as_int(at)] = REPLACE ? lane_sel<PathEq<m>::m>(diag, c[m]) : c[m];
   });
   wsync();
 }
@@ -65,7 +65,7 @@ __device__ __forceinline__ void unpack_L(const Sim& s, float (&c)[PP], int pd, i
   const int lane = opaque_lane(lane_);
   static_for<0, PP, 1>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
-    const float x = s.L[m < 12 || lane >= 32 ? path_packed<m>(pd, lane) : 0];
+    const float x = s.u.nt.L[m < 12 || lane >= 32 ? path_packed<m>(pd, lane) : 0];
     c[m] = m < 12 ? lane_sel0<PATH_VALID>(x) : lane_sel0<PATH_ARMS>(x);
   });
   wsync();
@@ -96,13 +96,27 @@ __device__ __forceinline__ void dof_motion(const Sim& s, int i, float* w, float*
   }
 }
 
-// Entry t of a chain-table row (the dofs moving a body, ascending; padding 255) for the row of dof `lane`, clamped to
-// lane: a chain's entries are lane's ancestor dofs and lane itself, so the clamp maps the padding and a root dof past
-// lane (the root rows' chains hold all 6 root dofs) to the diagonal. A row assembly then stores every entry
-// unconditionally: the clamped ones store the diagonal's value again.
-__device__ __forceinline__ int chain_dof_row(const unsigned* ch, int t, int lane) {
-  return (int)min((ch[t >> 2] >> (8 * (t & 3))) & 255u, (unsigned)lane);
+// Entry t of the chain of the body of dof `lane` (its ancestor dofs and itself, ascending: the root's 6, then the path's
+// as lanes of the path layout run, t + 0 / 6 / 12 / 19), clamped to lane: past the chain's end, and for a root dof past
+// lane, the diagonal. A row assembly then stores every entry unconditionally: the clamped ones store the diagonal's
+// value again.
+__device__ __forceinline__ int chain_dof_row(int t, int lane) {
+  const int o6 = lane < 12 ? 0 : lane < 18 ? 6 : 12, o9 = lane < 28 ? o6 : 19;
+  return min(t + (t < 6 ? 0 : t < 9 ? o6 : o9), lane);
 }
+constexpr bool check_chain_rows() {  // the entries are the ancestor dofs
+  for (int i = 0; i < NV; i++) {
+    const int o6 = i < 12 ? 0 : i < 18 ? 6 : 12, o9 = i < 28 ? o6 : 19;
+    uint64_t m = 0;
+    for (int t = 0; t < MAXCHAIN; t++) {
+      const int j = t + (t < 6 ? 0 : t < 9 ? o6 : o9);
+      m |= (uint64_t)1 << (j < i ? j : i);
+    }
+    if (m != TREE.dofanc[i]) return false;
+  }
+  return true;
+}
+static_assert(check_chain_rows(), "chain_dof_row");
 
 // (n, f) = I (w, v) for a packed spatial inertia about O: n = J w + h x v, f = m v - h x w (source.py:305-313)
 __device__ __forceinline__ void apply_inertia(const float* J, const float* w, const float* v, float* n, float* f) {
@@ -116,7 +130,7 @@ __device__ __forceinline__ void apply_inertia(const float* J, const float* w, co
 }
 
 // (M + dg diag(kv))^-1 b on the dof lanes, b an LDS vector over the dofs (36 words); the factor's rows are left in c
-// (and s.pf), its diagonal in *diag
+// (and s.u.nt.pf), its diagonal in *diag
 __device__ __forceinline__ float solve_M(Sim& s, float dg, const float* b, int pd, int lane, float (&c)[PP], float* diag) {
   const PathRow row = path_row(s.M[pd], s.M[NV], lane);
   const float dv = lane_sel0<PATH_VALID>(s.M[pd][pd] + dg * cKv[min(pd, NV - 1)]);
@@ -125,11 +139,12 @@ __device__ __forceinline__ float solve_M(Sim& s, float dg, const float* b, int p
     c[m] = path_entry<m>(row);
     if (dg != 0.f) c[m] = lane_sel<PathEq<m>::m>(dv, c[m]);
   });
-  *diag = path_factor(c, s.pf, lane);
-  return dof_value(path_solve(s.pf, c, *diag, path_value(b, pd), lane), lane);
+  *diag = path_factor(c, s.u.nt.pf, lane);
+  return dof_value(path_solve(s.u.nt.pf, c, *diag, path_value(b, pd), lane), lane);
 }
 
-__device__ void smooth(Sim& s, int pd, int lane) {
+// returns qacc_smooth on the dof lanes
+__device__ float smooth(Sim& s, int pd, int lane) {
   // each hinge body's local transform, one lane per body: q_l = quat (x) hinge rotation, the body's offset in its
   // parent's frame p_b, and the hinge axis in the parent's frame a_l = quat a (the hinge rotation keeps its own axis)
   if (lane >= 2 && lane < NB) {
@@ -145,8 +160,7 @@ __device__ void smooth(Sim& s, int pd, int lane) {
   }
   wsync();
   // FK: each body lane walks its own chain from the root: pose, velocity, and the bias acceleration (qacc = 0;
-  // gravity as the root's -g) (source.py:186-235 fwd_body). The chain's bodies come from the LDS chain table (the
-  // hinge dofs past the root's 6, body = dof - 4), their local transforms from the table above.
+  // gravity as the root's -g) (source.py:186-235 fwd_body); the bodies' local transforms from the table above.
   float Q[4], X[3], W[3], V[3], AL[3], A[3];
   {
     float n = rsqrtf(s.qpos[3] * s.qpos[3] + s.qpos[4] * s.qpos[4] + s.qpos[5] * s.qpos[5] + s.qpos[6] * s.qpos[6]);
@@ -154,15 +168,16 @@ __device__ void smooth(Sim& s, int pd, int lane) {
     for (int k = 0; k < 3; k++) { X[k] = s.qpos[k]; V[k] = s.qvel[k]; A[k] = -kGrav[k]; AL[k] = 0.f; }
     qrot(Q, s.qvel + 3, W);
   }
+  // the body at depth l + 1 on the lane's chain, up to the lane's own: its path's (PATHS; bodies ascend along a path)
   const int b = lane < NB ? lane : 0;
-  unsigned ch[4];
-  for (int k = 0; k < 4; k++) ch[k] = s.chain[b][k];
+  const int plo = b >= 14 ? 14 : b >= 8 ? 8 : 2, phi = b >= 24 ? 21 : b >= 14 ? 14 : plo;
+  static_assert(PATHS.lo[0] == 2 && PATHS.lo[1] == 8 && PATHS.lo[2] == 14 && PATHS.hi[2] == 14 && PATHS.hi[3] == 21,
+                "the paths of the FK walk");
 #pragma unroll
   for (int l = 1; l < MAXDEPTH; l++) {
-    bool on;
-    const int d = chain_dof(ch, 5 + l, &on);  // the hinge dof of the body at depth l + 1 on b's chain
-    if (on) {
-      const int k = d - 4;
+    const int k = (l <= 3 ? plo : phi) + l - 1;
+    if (k <= b) {
+      const int d = k + 4;
       const float* h = s.u.sm.hl[k];
       const float ql[4] = {h[0], h[1], h[2], h[3]}, pb[3] = {h[4], h[5], h[6]}, al[3] = {h[8], h[9], h[10]};
       float t[3], aw[3], awd[3], u[3], wr[3], u2[3], q1[4];
@@ -280,12 +295,10 @@ __device__ void smooth(Sim& s, int pd, int lane) {
     // M[i][j] = S_j . I_c(body i) S_i on the chain of dof i's body (its ancestor dofs j <= i), both halves; the
     // rest of M is zero (zero-filled above, earlier in this wave's LDS order). Two lanes never store the same entry:
     // lane i writes row i and column i at j <= i (the entry (i, i) twice)
-    unsigned ch[4];
-    for (int k = 0; k < 4; k++) ch[k] = s.chain[bi][k];
     const float arm = cArm[lane];
 #pragma unroll
     for (int t = 0; t < MAXCHAIN; t++) {
-      const int j = chain_dof_row(ch, t, lane);
+      const int j = chain_dof_row(t, lane);
       const float mij = s.S[j][0] * n[0] + s.S[j][1] * n[1] + s.S[j][2] * n[2] + s.S[j][4] * f[0] + s.S[j][5] * f[1]
                         + s.S[j][6] * f[2] + (j == lane ? arm : 0.f);
       s.M[lane][j] = mij;  // j <= lane: both halves (the clamped entries store the diagonal again)
@@ -312,8 +325,8 @@ __device__ void smooth(Sim& s, int pd, int lane) {
   // qacc_smooth = M^-1 qfrc_smooth
   float c[PP], diag;
   const float x = solve_M(s, 0.f, s.qsm, pd, lane, c, &diag);
-  if (lane < NV) s.qacc0[lane] = x;
   wsync();
+  return x;
 }
 
 }  // namespace g1k
@@ -357,12 +370,10 @@ __device__ void collision(Sim& s, int lane) {
     for (int e = 0; e < 2; e++) {
       const int idx = off + (e == 1 ? (int)o.has[0] : 0);
       if (o.has[e] && idx < MAXCON) {
-        float* st = s.u.col.stage[idx];
-        st[0] = o.d[e];
-        for (int k = 0; k < 3; k++) st[1 + k] = o.pos[e][k];
-        for (int k = 0; k < 9; k++) st[4 + k] = o.fr[e][k];
-        st[13] = __int_as_float(pr);
-        st[14] = __int_as_float(o.slot[e]);
+        float4* st = reinterpret_cast<float4*>(s.u.col.stage[idx]);  // the second tangent is n x b (make_frame)
+        st[0] = make_float4(o.d[e], o.pos[e][0], o.pos[e][1], o.pos[e][2]);
+        st[1] = make_float4(o.fr[e][0], o.fr[e][1], o.fr[e][2], o.fr[e][3]);
+        st[2] = make_float4(o.fr[e][4], o.fr[e][5], __int_as_float(pr | o.slot[e] << 16), 0.f);
       }
     }
     total += tn;
@@ -408,15 +419,14 @@ __device__ __forceinline__ void kbimp(float pos, float* k, float* b, float* imp)
 // the leaves (PATHS), lane c < 6 of a group carrying component c: the sums of each body's chain in its order, 10 steps
 // of 2 loads, an FMA and a store, every address a per-lane base plus a compile-time offset. Both arm groups compute
 // the waist's bodies (the same values); the legs' groups run 4 steps past their 6 bodies, and lanes c >= 6 every
-// step, into a sink (the Hessian's self-contact staging, unused outside the Hessian). The world body gets 0.
+// step, into the rows' unused places 3 and 7. The world body gets 0.
 __device__ __forceinline__ void body_vel(Sim& s, const float* v, int lane) {
   const int g = lane >> 4, c = lane & 15;
   const bool comp = c < 6;
   const int so = comp ? (c < 3 ? c : c + 1) : 0;  // the component's place in a row of S and bw: w 0..2, v 4..6
   const int lo = g == 0 ? PATHS.lo[0] : g == 1 ? PATHS.lo[1] : g == 2 ? PATHS.lo[2] : PATHS.lo[3];
   const int hi = g == 0 ? PATHS.hi[0] : g == 1 ? PATHS.hi[1] : g == 2 ? PATHS.hi[2] : PATHS.hi[3];
-  float* sink = &s.u.nt.psi[0][0] + (lane & 7);  // 8 * PATH_STEPS + 7 floats: inside psi
-  static_assert(8 * PATH_STEPS + 8 <= 4 * SELF_CHUNK * 8, "the sink inside psi");
+  float* sink = &s.u.nt.bw[hi][lane & 1 ? 3 : 7];
   const float rw = s.S[3][so] * v[3] + s.S[4][so] * v[4] + s.S[5][so] * v[5];
   float T = c < 3 ? rw : v[comp ? c - 3 : 0];
   (comp && g < 2 ? &s.u.nt.bw[1 - g][so] : sink)[0] = g == 0 ? T : 0.f;  // the root body; the world body 0
@@ -484,7 +494,7 @@ __device__ __forceinline__ float matvec(const Sim& s, const float* v, int lane_)
 }
 
 // ============================================================================================== Newton
-// fresh: the factor is H's at the final zones; pattern, diag: where it is (0: s.pf and diag, else s.L)
+// fresh: the factor is H's at the final zones; pattern, diag: where it is (0: s.u.nt.pf and diag, else s.L)
 struct NewtonOut { int it, pattern; float diag; bool conv, fresh; };
 
 // The floor contacts are the contact lanes [0, nf) sorted by body (the floor pairs come first in pair order, sorted by
@@ -568,7 +578,7 @@ __device__ float newton_grad(Sim& s, const Rows& R, int lane, bool con) {
 
 __device__ __forceinline__ float lane_cost(const Sim& s, const Rows& R, int lane) {
   float g = 0.f;
-  if (lane < NV) g = 0.5f * (s.Ma[lane] - s.qsm[lane]) * (s.qacc[lane] - s.qacc0[lane]);
+  if (lane < NV) g = 0.5f * (s.Ma[lane] - s.qsm[lane]) * (s.qacc[lane] - R.a0);
 #pragma unroll
   for (int t = 0; t < 4; t++)
     if (t < R.nr && R.jar[t] < 0.f) g += 0.5f * R.D * R.jar[t] * R.jar[t];
@@ -622,7 +632,7 @@ __device__ __forceinline__ void contact_stiffness(const Rows& R, const float* dd
   K[15] = Kf[0][0]; K[16] = Kf[1][1]; K[17] = Kf[2][2]; K[18] = Kf[0][1]; K[19] = Kf[0][2]; K[20] = Kf[1][2];
 }
 
-// s.L += the contacts between robot bodies selfm (lanes), sum over the active pyramid edges t of u_t u_t' with u_t =
+// s.u.nt.L += the contacts between robot bodies selfm (lanes), sum over the active pyramid edges t of u_t u_t' with u_t =
 // sqrt(D) J' e_t, u_t[i] = sigma_i S_i . (r x e_t, e_t), sigma_i = (dof i moves body 2) - (dof i moves body 1). On the
 // matrix cores (v_mfma_f32_16x16x4f32: lane l gives A[l % 16][l / 16] and B[l / 16][l % 16], holds C[4 (l / 16) + e]
 // [l % 16]), a batch of SELF_BATCH contacts at a time, its 16 edge vectors psi = (r x e_t, e_t) in LDS with row
@@ -655,12 +665,12 @@ __device__ __forceinline__ void add_self_contacts(Sim& s, const Rows& R, const f
   float H[3][3][4];
   auto tiles = [&](auto f) {
     const int ln = opaque_lane(lane), r = ln & 15, k = ln >> 4;
-    float* const sink = s.L + LSINK + ln;
+    float* const sink = s.u.nt.L + LSINK + ln;
     static_for<0, 3, 1>([&](auto ic) {
       static_for<0, 4, 1>([&](auto ec) {
         constexpr int ti = decltype(ic)::value, e = decltype(ec)::value;
         if constexpr (16 * ti + e < NV) {
-          float* const row = s.L + tri(16 * ti + 4 * k + e, 0) + r;
+          float* const row = s.u.nt.L + tri(16 * ti + 4 * k + e, 0) + r;
           static_for<0, ti + 1, 1>([&](auto jc) {
             constexpr int tj = decltype(jc)::value;
             const bool in = (ti < 2 || k == 0) && (ti != tj || r <= 4 * k + e);
@@ -674,16 +684,20 @@ __device__ __forceinline__ void add_self_contacts(Sim& s, const Rows& R, const f
   for (unsigned long long m = selfm; m;) {
     const int q = prefix_count(m, lane);
     if (((m >> lane) & 1ull) && q < SELF_CHUNK) {  // this contact's 4 edge rows: sqrt(D) (r x e_t, e_t), e_t = n +- mu t1, n +- mu t2
-      const float sd = sqrtf(R.D);
+      // (opaque values: what does not change over Newton's iterations is not formed ahead of them and held, 30 registers)
+      const float sd = sqrtf(opaque(R.D)), mu = opaque(R.mu);
+      float fr[9], rr[3];
+      for (int k = 0; k < 9; k++) fr[k] = opaque(R.fr[k]);
+      for (int k = 0; k < 3; k++) rr[k] = opaque(R.r[k]);
 #pragma unroll
       for (int t = 0; t < 4; t++) {
         float e[3];
-        const float sg = (t & 1) ? -R.mu : R.mu;
-        const float* ta = R.fr + 3 * (1 + (t >> 1));
-        for (int k = 0; k < 3; k++) e[k] = R.dim == 3 ? R.fr[k] + sg * ta[k] : (t == 0 ? R.fr[k] : 0.f);
+        const float sg = (t & 1) ? -mu : mu;
+        const float* ta = fr + 3 * (1 + (t >> 1));
+        for (int k = 0; k < 3; k++) e[k] = R.dim == 3 ? fr[k] + sg * ta[k] : (t == 0 ? fr[k] : 0.f);
         const float sc = d[t] != 0.f ? sd : 0.f;
         float re[3];
-        cross(R.r, e, re);
+        cross(rr, e, re);
         float4* o = reinterpret_cast<float4*>(s.u.nt.psi[16 * (q >> 2) + 4 * t + (q & 3)]);
         o[0] = make_float4(sc * re[0], sc * re[1], sc * re[2], 0.f);
         o[1] = make_float4(sc * e[0], sc * e[1], sc * e[2], 0.f);
@@ -815,13 +829,14 @@ __device__ __forceinline__ int hessian(Sim& s, const Rows& R, int pd, int lane, 
 }
 
 
-__device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int pd, int lane, bool con, int iterations) {
+// factor: leave H's factor at the final zones, assembled once more when the last step changed a zone
+__device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int pd, int lane, bool con, int iterations, bool factor) {
   // warm start against qacc_smooth: keep the cheaper (step.py:1974-1988)
   refresh(s, R, lane, con);
   float cost = wsum(lane_cost(s, R, lane));
   float wq = lane < NV ? s.qacc[lane] : 0.f, wma = lane < NV ? s.Ma[lane] : 0.f, wj[4], wl = R.ljar;
   for (int t = 0; t < 4; t++) wj[t] = R.jar[t];
-  if (lane < NV) s.qacc[lane] = s.qacc0[lane];
+  if (lane < NV) s.qacc[lane] = R.a0;
   wsync();
   refresh(s, R, lane, con, true);
   const float cost0 = wsum(lane_cost(s, R, lane));
@@ -834,10 +849,12 @@ __device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int pd, int lane, b
     cost = cost0;
   }
   newton_grad(s, R, lane, con);
-  int it = 0, pattern = 0;  // pattern: where H's factor is (0: s.pf and diag, else s.L)
+  int it = 0, pattern = 0;  // pattern: where H's factor is (0: s.u.nt.pf and diag, else s.L)
   float diag = 1.f;
   bool conv = false, zsame = false;
-  while (it < iterations) {
+  for (;;) {
+    const bool done = conv || it >= iterations;
+    if (done && (zsame || !factor)) break;
     // a compiler barrier: LDS values are loaded where they are used inside the iteration, not hoisted out of the loop
     // into registers held across all of it
     asm volatile("" ::: "memory");
@@ -846,14 +863,15 @@ __device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int pd, int lane, b
     if (!zsame) {  // else no row changed its zone in the last step: H, and so its factor, are unchanged
       pattern = hessian(s, R, pd, lane, con, c);
       PROF(PH_HESS);
-      if (pattern == 0) diag = path_factor(c, s.pf, lane);
+      if (pattern == 0) diag = path_factor(c, s.u.nt.pf, lane);
       else factor_L(s, lane, pattern);
       PROF(PH_FACTOR);
+      if (done) break;
     } else if (pattern == 0) {
-      path_load(s.pf, c, lane);
+      path_load(s.u.nt.pf, c, lane);
     }
-    if (pattern == 0) p = dof_value(path_solve(s.pf, c, diag, -path_value(s.grad, pd), lane), lane);
-    else p = ltl_solve(s.L, lane < NV ? -s.grad[lane] : 0.f, lane);
+    if (pattern == 0) p = dof_value(path_solve(s.u.nt.pf, c, diag, -path_value(s.grad, pd), lane), lane);
+    else p = ltl_solve(s.u.nt.L, lane < NV ? -s.grad[lane] : 0.f, lane);
     PROF(PH_SOLVE);
 #ifdef G1_PROFILE
     if (lane == 0) s.prof_acc[PH_ITERS] += 1;
@@ -865,7 +883,6 @@ __device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int pd, int lane, b
     rows_jv(s, R, s.p, lane, con, jv, &ljv);
     PROF(PH_LSJV);
     const float mp = matvec(s, s.p, lane);
-    if (lane < NV) s.Mp[lane] = mp;
     // per row: x(alpha) = jar + alpha jv; rows past the kept ones start at +1e30 (never in the quadratic zone)
     float xr[5], vr[5], dr[5];
 #pragma unroll
@@ -954,7 +971,6 @@ __device__ __forceinline__ NewtonOut newton(Sim& s, Rows& R, int pd, int lane, b
     cost = newcost;
     it++;
     conv = improvement < kTol || kScale * gn < kTol;
-    if (conv) break;
   }
   return NewtonOut{it, pattern, diag, conv, it > 0 && zsame};
 }
@@ -979,7 +995,7 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
   }
   PROF(PH_TAPE);
   const int pd = path_lane_dof(lane);  // this lane's dof in the path layout (NV: none)
-  smooth(s, pd, lane);
+  R.a0 = smooth(s, pd, lane);
   PROF(PH_SMOOTH);
   collision(s, lane);
   PROF(PH_COLLIDE);
@@ -989,8 +1005,8 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
       unsigned e[2];
       for (int t = 0; t < 2; t++) {
         const int c = 2 * lane + t;
-        e[t] = c < nc ? ((unsigned)__float_as_int(s.u.col.stage[c][13]) | (unsigned)__float_as_int(s.u.col.stage[c][14]) << 9)
-                      : TAPE_CON_NONE;
+        const unsigned ps = (unsigned)__float_as_int(s.u.col.stage[c][10]);
+        e[t] = c < nc ? ((ps & 0xFFFFu) | (ps >> 16) << 9) : TAPE_CON_NONE;
       }
       rec[REC_CON + lane] = __uint_as_float(e[0] | e[1] << 16);
     }
@@ -1005,11 +1021,13 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
   for (int k = 0; k < 9; k++) R.fr[k] = 0.f;
   float dist = 0.f, piw = 0.f;
   if (con) {
-    const float* st = s.u.col.stage[lane];
-    dist = st[0];
-    for (int k = 0; k < 3; k++) R.r[k] = st[1 + k] - s.O[k];
-    for (int k = 0; k < 9; k++) R.fr[k] = st[4 + k];
-    pair = __float_as_int(st[13]);
+    const float4* st = reinterpret_cast<const float4*>(s.u.col.stage[lane]);
+    const float4 x0 = st[0], x1 = st[1], x2 = st[2];
+    dist = x0.x;
+    R.r[0] = x0.y - s.O[0]; R.r[1] = x0.z - s.O[1]; R.r[2] = x0.w - s.O[2];
+    R.fr[0] = x1.x; R.fr[1] = x1.y; R.fr[2] = x1.z; R.fr[3] = x1.w; R.fr[4] = x2.x; R.fr[5] = x2.y;
+    cross(R.fr, R.fr + 3, R.fr + 6);
+    pair = __float_as_int(x2.z) & 0xFFFF;
     const PairC pc = cPair[pair];
     const PairRow prow = cPairRow[pair];
     const unsigned w = pc.w;
@@ -1079,21 +1097,17 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
     }
     sing = ballot(nu < SINGULAR_NU) != 0ull;
   }
-  NewtonOut no = newton(s, R, pd, lane, con, iterations);
+  const NewtonOut no = newton(s, R, pd, lane, con, iterations, rec != nullptr);
   PROF(PH_NINIT);
   if (lane == 0) s.niter = no.it;
   if (rec) {  // the final zones, and H's factor at them (assembled again when the last step changed a zone)
-    float c[PP];
-    if (!no.fresh) {
-      no.pattern = hessian(s, R, pd, lane, con, c);
-      if (no.pattern == 0) no.diag = path_factor(c, s.pf, lane);
-      else factor_L(s, lane, no.pattern);
-    } else if (no.pattern == 0) {
-      path_load(s.pf, c, lane);
+    if (no.pattern == 0) {
+      float c[PP];
+      path_load(s.u.nt.pf, c, lane);
       wsync();
+      pack_L<true>(s, c, no.diag, pd, lane);
     }
-    if (no.pattern == 0) pack_L<true>(s, c, no.diag, pd, lane);
-    tape_put(rec + REC_LH, s.L, NTRI, REC_LQ - REC_LH, lane);
+    tape_put(rec + REC_LH, s.u.nt.L, NTRI, REC_LQ - REC_LH, lane);
     unsigned cz = 0u;
     for (int t = 0; t < 4; t++) cz |= (t < R.nr && R.jar[t] < 0.f) ? 1u << t : 0u;
     // 4 bits per contact: lanes 8 w .. 8 w + 7 into word w (gathered by shuffles)
@@ -1137,9 +1151,9 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
       // are written into the factor's zeros in LDS first (s.L is factored afresh before its next use); a position's
       // fourth word, which nothing writes in s.X, as 0
       for (int q = lane; q < POSE_WORDS; q += WL)
-        s.L[cPoseSlots.pos[q]] = q >= 4 * NB && (q & 3) == 3 ? 0.f : (&s.Q[0][0])[q];
+        s.u.nt.L[cPoseSlots.pos[q]] = q >= 4 * NB && (q & 3) == 3 ? 0.f : (&s.Q[0][0])[q];
       wsync();
-      tape_put(rec + REC_LQ, s.L, NTRI, REC_ADJCOST - REC_LQ, lane);
+      tape_put(rec + REC_LQ, s.u.nt.L, NTRI, REC_ADJCOST - REC_LQ, lane);
       if (lane < REC_LH - REC_AADV) rec[REC_AADV + lane] = lane < NV ? adv : 0.f;
     }
     wsync();
@@ -1190,16 +1204,27 @@ __device__ __forceinline__ void set_priority_by_remaining(unsigned long long t_s
   else __builtin_amdgcn_s_setprio(0);
 }
 
-// one world per wave64 (one workgroup of 64 lanes)
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_forward(int nw, const float* __restrict__ qpos, const float* __restrict__ qvel,
-                                                const float* __restrict__ warm, const float* __restrict__ ctrl,
-                                                const float* __restrict__ fric, const float* __restrict__ com,
-                                                int iterations, int nsub, float* __restrict__ oqpos,
-                                                float* __restrict__ oqvel, float* __restrict__ owarm,
-                                                int* __restrict__ info, float* __restrict__ ocon,
-                                                float* __restrict__ tape, const int* __restrict__ perm,
-                                                unsigned long long* __restrict__ diag) {
-  __shared__ Sim s;
+struct ForwardArgs {
+  int nw;
+  const float *qpos, *qvel, *warm, *ctrl, *fric, *com;
+  int iterations, nsub;
+  float *oqpos, *oqvel, *owarm;
+  int* info;
+  float *ocon, *tape;
+  const int* perm;
+  unsigned long long* diag;
+};
+
+// one world on this wave64 (a workgroup of 64 lanes)
+__device__ __forceinline__ void forward_world(Sim& s, const ForwardArgs& A) {
+  const int nw = A.nw, iterations = A.iterations, nsub = A.nsub;
+  const float *__restrict__ qpos = A.qpos, *__restrict__ qvel = A.qvel, *__restrict__ warm = A.warm;
+  const float *__restrict__ ctrl = A.ctrl, *__restrict__ fric = A.fric, *__restrict__ com = A.com;
+  float *__restrict__ oqpos = A.oqpos, *__restrict__ oqvel = A.oqvel, *__restrict__ owarm = A.owarm;
+  int* __restrict__ info = A.info;
+  float *__restrict__ ocon = A.ocon, *__restrict__ tape = A.tape;
+  const int* __restrict__ perm = A.perm;
+  unsigned long long* __restrict__ diag = A.diag;
   const int lane = threadIdx.x;
   if ((int)blockIdx.x >= nw) return;
   const int w = perm ? perm[blockIdx.x] : (int)blockIdx.x;  // heaviest worlds first (g1_order.hip)
@@ -1215,7 +1240,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   if (lane == 0) { s.fric = ifr; s.flags = 0; s.niter = 0; s.dcnt = 0; s.acost = 0; }
   s.dsub[lane] = lane < NV ? cTree.dofmask32[lane] : 0u;
   if (lane < 8) s.S[NV][lane] = 0.f;
-  chain_table(s.chain, lane);
 #ifdef G1_PROFILE
   if (lane < NPHASE) s.prof_acc[lane] = 0;
   if (lane == 0) {
@@ -1264,10 +1288,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   }
 }
 
+// Two builds of the kernel, the same results. k_forward: two waves per SIMD with registers to spare (190), the shortest
+// chain of a world by itself. k_forward3: three waves per SIMD (168 registers, 26 values in scratch, outside Newton's
+// loop but for a few loads; 14 KB of LDS, 11 worlds per CU): two waves leave a quarter of the SIMD's issue slots empty
+// (63 k VALU instructions a world-step in 168 k slots of its wave), the third fills them, and a world by itself takes 2%
+// longer. Forward of standing / contact-heavy worlds in us, two waves against three: 2048 550 / 508 against 563 / 516,
+// 2304 483 / 517 against 499 / 533, 2560 533 / 581 against 500 / 539, 3072 602 / 665 against 513 / 556, 4096 705 / 742
+// against 673 / 729, 16384 2353 / 2560 against 2000 / 2184: three waves from more than 9 worlds a CU on.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_forward(ForwardArgs A) {
+  __shared__ Sim s;
+  forward_world(s, A);
+}
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_forward3(ForwardArgs A) {
+  __shared__ Sim s;
+  forward_world(s, A);
+}
+constexpr int WAVES3_WORLDS_PER_CU = 9;  // beyond so many worlds a CU: k_forward3
+
 }  // namespace g1k
 
 namespace g1k {
 int launch_order_fwd(hipStream_t st, int nw, const float* qpos, void* work);
+int worlds_of_cus(int per_cu);
 int resident_worlds();
 // order: 0 index order (work unused), 1 compute the order into work first (index order when the batch fits the
 // GPU's resident slots at once: the order cannot change the makespan there), 2 the order already in work; diag: the
@@ -1285,8 +1327,9 @@ int launch_forward(hipStream_t st, int nw, const float* qpos, const float* qvel,
     }
     perm = (const int*)work;
   }
-  hipLaunchKernelGGL(k_forward, dim3(nw), dim3(64), 0, st, nw, qpos, qvel, warm, ctrl, fric, com, iterations, nsub,
-                     oq, ov, ow, info, ocon, tape, perm, diag);
+  const ForwardArgs A{nw, qpos, qvel, warm, ctrl, fric, com, iterations, nsub, oq, ov, ow, info, ocon, tape, perm, diag};
+  if (nw > worlds_of_cus(WAVES3_WORLDS_PER_CU)) hipLaunchKernelGGL(k_forward3, dim3(nw), dim3(64), 0, st, A);
+  else hipLaunchKernelGGL(k_forward, dim3(nw), dim3(64), 0, st, A);
   return (int)hipGetLastError();
 }
 size_t forward_lds_bytes() { return sizeof(Sim); }

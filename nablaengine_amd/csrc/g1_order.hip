@@ -28,23 +28,23 @@ namespace g1k {
 
 constexpr int NBKT = COST_BUCKETS;
 
-// worlds resident at once on the current device: 8 per CU (the forward's and the adjoint's LDS and VGPRs), the CU
-// count queried once per device (host threads may race to store the same value: atomics); 0 when the query fails
-// (the order is then always computed)
+// per_cu worlds on every CU of the current device, the CU count queried once per device (host threads may race to
+// store the same value: atomics); 0 when the query fails
 constexpr int WORLDS_PER_CU = 8, MAX_DEVICES = 64;
-int resident_worlds() {
-  static std::atomic<int> per_dev[MAX_DEVICES];  // 0: not queried yet
+int worlds_of_cus(int per_cu) {
+  static std::atomic<int> cus_of[MAX_DEVICES];  // 0: not queried yet
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 0;
-  int n = per_dev[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    int cus = 0;
+  int cus = cus_of[dev].load(std::memory_order_relaxed);
+  if (cus == 0) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 0;
-    n = WORLDS_PER_CU * cus;
-    per_dev[dev].store(n, std::memory_order_relaxed);
+    cus_of[dev].store(cus, std::memory_order_relaxed);
   }
-  return n;
+  return per_cu * cus;
 }
+// a batch up to this size is resident at once: 8 worlds per CU (two waves per SIMD, the adjoint's and k_forward's); 0
+// when the CU count is not known (the order is then always computed)
+int resident_worlds() { return worlds_of_cus(WORLDS_PER_CU); }
 
 // contacts at the input state: FK of body poses (each body lane walks its chain from the root), geom poses, the main
 // kernel's broadphase and narrowphase (the same code); the cost counts the contacts' constraint rows (4 per pyramid
