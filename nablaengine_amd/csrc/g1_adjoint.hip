@@ -14,6 +14,7 @@
 // bodies in body order); no atomics.
 #include "g1_collide.h"
 #include "g1_diag.h"
+#include "g1_path.h"
 #include "g1_tape.h"
 
 namespace g1k {
@@ -64,7 +65,7 @@ __device__ __forceinline__ Sv ld_sv(const float* p) {
 }
 
 enum { TW_V = 0, TW_L, TW_Y, TW_AW, TW_A2, TW_A1, NTW };  // per-body twists
-enum { FB_F1 = 0, FB_P, FB_X1, FB_F2, FB_P2, FB_EG, FB_OL, FB_OA, FB_OV, NFB };  // per-body force vectors
+enum { FB_F1 = 0, FB_P, FB_X1, FB_F2, FB_P2, FB_EG, FB_OL, FB_OA, NFB };  // per-body force vectors
 __device__ __forceinline__ Sv ld_sv6(const float* p) {  // a spatial vector packed as 6 floats (8-byte aligned)
   Sv r;
   for (int k = 0; k < 3; k++) { r.w[k] = p[k]; r.v[k] = p[3 + k]; }
@@ -136,33 +137,36 @@ __device__ unsigned long long g_prof_adj[PROF_WORLDS][NPHASE];
 #define APROF(k) do { } while (0)
 #endif
 
-// impedance and its derivative in the distance (kbimp's curve, solimp power 2; 0 where the curve is clamped)
-__device__ __forceinline__ void imp_d(const float* solimp, float pos, float* imp, float* dimp) {
-  const float dmin = fminf(fmaxf(solimp[0], 1e-4f), 0.9999f), dmax = fminf(fmaxf(solimp[1], 1e-4f), 0.9999f);
-  const float width = fmaxf(1e-15f, solimp[2]), mid = fminf(fmaxf(solimp[3], 1e-4f), 0.9999f);
-  const float iwd = 1.f / width, x = fabsf(pos) * iwd, sg = pos < 0.f ? -1.f : 1.f;
+// impedance and its derivative in the distance (kbimp's curve, solimp power 2; 0 where the curve is clamped); solimp
+// and solref as compile-time values
+constexpr Arr<float, 2> aJSOLREF = to_float(JNT_SOLREF), aPSOLREF = to_float(PAIR_SOLREF);
+constexpr Arr<float, 5> aJSOLIMP = to_float(JNT_SOLIMP), aPSOLIMP = to_float(PAIR_SOLIMP);
+static_assert(JNT_SOLIMP[4] == 2.0 && PAIR_SOLIMP[4] == 2.0, "imp_d assumes the solimp power 2");
+constexpr float amax(float a, float b) { return a < b ? b : a; }
+constexpr float aclamp(float x) { return x < 1e-4f ? 1e-4f : x > 0.9999f ? 0.9999f : x; }
+template <const Arr<float, 5>& SOLIMP>
+__device__ __forceinline__ void imp_d(float pos, float* imp, float* dimp) {
+  constexpr float dmin = aclamp(SOLIMP.v[0]), dmax = aclamp(SOLIMP.v[1]);
+  constexpr float width = amax(1e-15f, SOLIMP.v[2]), mid = aclamp(SOLIMP.v[3]);
+  constexpr float iwd = 1.f / width, im0 = 1.f / mid, im1 = 1.f / (1.f - mid);
+  const float x = fabsf(pos) * iwd, sg = pos < 0.f ? -1.f : 1.f;
   *dimp = 0.f;
   if (x <= 0.f) { *imp = dmin; return; }
   if (x >= 1.f) { *imp = dmax; return; }
   float y, dy;
-  if (x <= mid) { const float im = 1.f / mid; y = x * x * im; dy = 2.f * x * im; }
-  else { const float im = 1.f / (1.f - mid); y = 1.f - (1.f - x) * (1.f - x) * im; dy = 2.f * (1.f - x) * im; }
+  if (x <= mid) { y = x * x * im0; dy = 2.f * x * im0; }
+  else { y = 1.f - (1.f - x) * (1.f - x) * im1; dy = 2.f * (1.f - x) * im1; }
   const float v = dmin + y * (dmax - dmin);
   if (v < dmin || v > dmax) { *imp = fminf(fmaxf(v, dmin), dmax); return; }
   *imp = v;
   *dimp = dy * (dmax - dmin) * sg * iwd;
 }
-__device__ __forceinline__ void kb_consts(const float* solref, const float* solimp, float* k, float* b) {
-  const float tc = fmaxf(solref[0], 2.f * kH), dr = solref[1];
-  const float dmax = fminf(fmaxf(solimp[1], 1e-4f), 0.9999f);
-  *k = 1.f / fmaxf(1e-15f, dmax * dmax * tc * tc * dr * dr);
-  *b = 2.f / fmaxf(1e-15f, dmax * tc);
+template <const Arr<float, 2>& SOLREF, const Arr<float, 5>& SOLIMP>
+__device__ __forceinline__ void kb_consts(float* k, float* b) {
+  constexpr float tc = amax(SOLREF.v[0], 2.f * kH), dr = SOLREF.v[1], dmax = aclamp(SOLIMP.v[1]);
+  *k = 1.f / amax(1e-15f, dmax * dmax * tc * tc * dr * dr);
+  *b = 2.f / amax(1e-15f, dmax * tc);
 }
-
-__constant__ inline Arr<float, 2> caJSolref = to_float(JNT_SOLREF);
-__constant__ inline Arr<float, 5> caJSolimp = to_float(JNT_SOLIMP);
-__constant__ inline Arr<float, 2> caPSolref = to_float(PAIR_SOLREF);
-__constant__ inline Arr<float, 5> caPSolimp = to_float(PAIR_SOLIMP);
 
 // the normal derivative's factor kappa(nu): 1 / nu exact (0), frozen (1), 1 / max(nu, eps) (2), frozen below eps (3)
 __device__ __forceinline__ float kappa(float nu, int normal) {
@@ -548,8 +552,25 @@ __device__ __forceinline__ void adj_integrator(Adj& s, int lane) {
   wsync();
 }
 
+// the pairs with the floor come first in the pair table
+constexpr int floor_pairs() {
+  int n = 0;
+  while (n < NPAIR && GEOM_BODY[PAIR_G1[n]] == 0) n++;
+  return n;
+}
+// whether the record's H, and so its factor, has the tree's sparsity: no row of a contact between two robot bodies was
+// in its quadratic zone
+__device__ __forceinline__ bool tree_sparse(const Adj& s, int lane) {
+  const unsigned zc = (s.czone[lane >> 3] >> (4 * (lane & 7))) & 15u;
+  return ballot(lane < s.ncon && zc != 0u && (s.con[lane] & 511u) >= (unsigned)floor_pairs()) == 0ull;
+}
+
 // y = Q^-1 a_adv bar (L_Q), a* bar = a_adv bar - h kv y; lambda = H^-1 a* bar (L_H)
 // clear: L_Q's frame slots set to 0 first (a copy of the factors made after the record's, whose frames were taken)
+// L_Q always, and L_H where no contact between two robot bodies was active, by the path layout's solves (about 140 vector
+// instructions where the solve one dof at a time takes 290; bitwise its result). Bound by vector issue: with the
+// compile-time impedance terms and the wrench sums' third left out below, k_adjoint went from 511 to 485 us at 16384
+// worlds, k_adjoint_sets from 1220 to 1150 us for the Jacobians of 600.
 __device__ __forceinline__ void adj_solves(Adj& s, int lane, bool clear) {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the factors' copies have landed in LDS
   wsync();
@@ -557,13 +578,20 @@ __device__ __forceinline__ void adj_solves(Adj& s, int lane, bool clear) {
     clear_pose_slots(s, lane);
     wsync();
   }
-  const float aab = lane < NV ? kH * s.vt[lane] : 0.f;
-  const float y = ltl_solve(s.lt.q, aab, lane);
-  if (lane < NV) s.y[lane] = y;
-  wsync();
-  const float asb = lane < NV ? aab - kH * cKv[lane] * y : 0.f;
-  const float lam = ltl_solve(s.lt.h, asb, lane);
-  if (lane < NV) s.lam[lane] = lam;
+  // in the path layout (g1_path.h): lane's dof pd, every value on each lane of its dof
+  const int pd = path_lane_dof(lane), pc = min(pd, NV - 1);
+  const float aab = lane_sel0<PATH_VALID>(kH * s.vt[pd]);
+  float y, lam;
+  path_solve_packed<1>(s.lt.q, pd, lane, &aab, &y);
+  if (pd < NV) s.y[pd] = y;  // the root's and the waist's several lanes hold the same value
+  const float asb = lane_sel0<PATH_VALID>(aab - kH * cKv[pc] * y);
+  if (tree_sparse(s, lane)) {
+    path_solve_packed<1>(s.lt.h, pd, lane, &asb, &lam);
+    if (pd < NV) s.lam[pd] = lam;
+  } else {
+    lam = ltl_solve(s.lt.h, lane_of(asb, owner_lane(min(lane, NV - 1))), lane);
+    if (lane < NV) s.lam[lane] = lam;
+  }
   wsync();
 }
 
@@ -581,15 +609,21 @@ __device__ __forceinline__ void adj_solves_sets(Adj& s, SetStage* st, int nc, in
     clear_pose_slots(s, lane);
     wsync();
   }
-  const float aab0 = lane < NV ? kH * st[0].vt[lane] : 0.f, aab1 = lane < NV && nc > 1 ? kH * st[1].vt[lane] : 0.f;
-  float y0, y1;
-  ltl_solve2(s.lt.q, aab0, aab1, lane, &y0, &y1);
-  if (lane < NV) { st[0].y[lane] = y0; st[1].y[lane] = y1; }
-  wsync();
-  const float asb0 = lane < NV ? aab0 - kH * cKv[lane] * y0 : 0.f, asb1 = lane < NV ? aab1 - kH * cKv[lane] * y1 : 0.f;
-  float l0, l1;
-  ltl_solve2(s.lt.h, asb0, asb1, lane, &l0, &l1);
-  if (lane < NV) { st[0].lam[lane] = l0; st[1].lam[lane] = l1; }
+  const int pd = path_lane_dof(lane), pc = min(pd, NV - 1);
+  const float kv = kH * cKv[pc];
+  float b[2] = {lane_sel0<PATH_VALID>(kH * st[0].vt[pd]), nc > 1 ? lane_sel0<PATH_VALID>(kH * st[1].vt[pd]) : 0.f}, x[2];
+  path_solve_packed<2>(s.lt.q, pd, lane, b, x);
+  if (pd < NV) { st[0].y[pd] = x[0]; st[1].y[pd] = x[1]; }
+#pragma unroll
+  for (int i = 0; i < 2; i++) b[i] = lane_sel0<PATH_VALID>(b[i] - kv * x[i]);
+  if (tree_sparse(s, lane)) {
+    path_solve_packed<2>(s.lt.h, pd, lane, b, x);
+    if (pd < NV) { st[0].lam[pd] = x[0]; st[1].lam[pd] = x[1]; }
+  } else {
+    const int own = owner_lane(min(lane, NV - 1));
+    ltl_solve2(s.lt.h, lane_of(b[0], own), lane_of(b[1], own), lane, &x[0], &x[1]);
+    if (lane < NV) { st[0].lam[lane] = x[0]; st[1].lam[lane] = x[1]; }
+  }
   wsync();
 }
 
@@ -730,8 +764,8 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
       const float q = s.qpos[lane + 1], dmin = q - cRange[2 * lane], dmax = cRange[2 * lane + 1] - q;
       const float sg = dmin < dmax ? 1.f : -1.f, pos = fminf(dmin, dmax);
       float k, b, imp, dimp;
-      kb_consts(caJSolref.v, caJSolimp.v, &k, &b);
-      imp_d(caJSolimp.v, pos, &imp, &dimp);
+      kb_consts<aJSOLREF, aJSOLIMP>(&k, &b);
+      imp_d<aJSOLIMP>(pos, &imp, &dimp);
       const float iw = cDinvw[lane];
       const float D = 1.f / fmaxf(iw * (1.f - imp) / imp, 1e-15f), dD = dimp / (iw * (1.f - imp) * (1.f - imp));
       const float jl = sg * s.lam[lane], x = sg * s.astar[lane] + k * imp * pos + b * sg * s.qvel[lane];
@@ -743,7 +777,6 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
   // contacts (lane = contact of the tape's table): replay, row terms, geometry VJP -> wrenches
   const int ncon = s.ncon;
   Sv cOmL = sv0(), cOmA = sv0(), cW1 = sv0(), cW2 = sv0();  // this lane's contact: row sums, the sides' wrenches
-  float cbb = 0.f;
   int cb1 = 0, cb2 = 0;
   bool cact = false;
   if (lane < ncon) {
@@ -768,8 +801,8 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
         for (int k = 0; k < 9; k++) fr[k] = which ? cd.fr[1][k] : cd.fr[0][k];
         const float mu = ((w >> 20) & 1u) ? s.fric : prow.mu;
         float k, b, imp, dimp;
-        kb_consts(caPSolref.v, caPSolimp.v, &k, &b);
-        imp_d(caPSolimp.v, dist, &imp, &dimp);
+        kb_consts<aPSOLREF, aPSOLIMP>(&k, &b);
+        imp_d<aPSOLIMP>(dist, &imp, &dimp);
         float iw = prow.iw;
         if (dim == 3) iw = (mu * mu * iw + iw) * 2.f * mu * mu / kImpratio;
         const float D = 1.f / fmaxf(iw * (1.f - imp) / imp, 1e-15f), dD = dimp / (iw * (1.f - imp) * (1.f - imp));
@@ -830,7 +863,6 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
         cOmA = OmA;
         cW1 = sv_add(G1, e1, -1.f);  // the b1 side's wrench (its twists enter with -)
         cW2 = sv_add(G2, e2);        // the b2 side's wrench
-        cbb = b;
         cact = true;
       }
     }
@@ -839,13 +871,14 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
   // per body: the contacts' wrenches and row sums (body 2 +, body 1 -); body lane B keeps its totals. The floor
   // contacts (body 1 the world) summed over the contact lanes once per distinct body they touch (masked wave sums,
   // a fixed order); a contact between two robot bodies taken one at a time, its values broadcast to every lane and
-  // added by the two body lanes (a wave sum per body it touches cost 24 sums of up to 6 steps each)
-  Sv EG = sv0(), OL = sv0(), OA = sv0(), OV = sv0();
+  // added by the two body lanes (a wave sum per body it touches costs 18 sums of up to 6 steps each)
+  Sv EG = sv0(), OL = sv0(), OA = sv0();
   const bool cself = cact && cb1 != 0;
+  const int nf = __popcll(ballot(lane < ncon && cb1 == 0));  // the floor contacts, the table's first
   for (unsigned m = wor(cact && !cself ? 1u << cb2 : 0u) & ~1u; m; m &= m - 1u) {
     const int B = __builtin_ctz(m);
     const bool on = cact && !cself && cb2 == B;
-    float x[24];
+    float x[18];
     for (int k = 0; k < 3; k++) {
       x[k] = on ? cW2.w[k] : 0.f;
       x[3 + k] = on ? cW2.v[k] : 0.f;
@@ -853,31 +886,25 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
       x[9 + k] = on ? cOmL.v[k] : 0.f;
       x[12 + k] = on ? cOmA.w[k] : 0.f;
       x[15 + k] = on ? cOmA.v[k] : 0.f;
-      x[18 + k] = on ? cbb * cOmA.w[k] : 0.f;
-      x[21 + k] = on ? cbb * cOmA.v[k] : 0.f;
     }
-    wsum_nw<24>(x, ncon);  // contact lanes only
+    wsum_nw<18>(x, nf);  // the floor contacts' lanes only
     if (lane == B)
       for (int k = 0; k < 3; k++) {
         EG.w[k] = x[k]; EG.v[k] = x[3 + k]; OL.w[k] = x[6 + k]; OL.v[k] = x[9 + k];
-        OA.w[k] = x[12 + k]; OA.v[k] = x[15 + k]; OV.w[k] = x[18 + k]; OV.v[k] = x[21 + k];
+        OA.w[k] = x[12 + k]; OA.v[k] = x[15 + k];
       }
   }
   for (unsigned long long m = ballot(cself); m; m &= m - 1ull) {
     const int c = __builtin_ctzll(m);
     const int b1 = rdli(cb1, c), b2 = rdli(cb2, c);
     const float s2 = lane == b2 ? 1.f : 0.f, s1 = lane == b1 ? 1.f : 0.f, sd = s2 - s1;
-    const float bb = rdl(cbb, c);
     for (int k = 0; k < 3; k++) {
       EG.w[k] += s2 * rdl(cW2.w[k], c) + s1 * rdl(cW1.w[k], c);
       EG.v[k] += s2 * rdl(cW2.v[k], c) + s1 * rdl(cW1.v[k], c);
       OL.w[k] += sd * rdl(cOmL.w[k], c);
       OL.v[k] += sd * rdl(cOmL.v[k], c);
-      const float aw = rdl(cOmA.w[k], c), av = rdl(cOmA.v[k], c);
-      OA.w[k] += sd * aw;
-      OA.v[k] += sd * av;
-      OV.w[k] += sd * (bb * aw);
-      OV.v[k] += sd * (bb * av);
+      OA.w[k] += sd * rdl(cOmA.w[k], c);
+      OA.v[k] += sd * rdl(cOmA.v[k], c);
     }
   }
   APROF(AP_BODYSUM);
@@ -896,12 +923,11 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
     st_sv6(s.fb[lane][FB_EG], EG);
     st_sv6(s.fb[lane][FB_OL], OL);
     st_sv6(s.fb[lane][FB_OA], OA);
-    st_sv6(s.fb[lane][FB_OV], OV);
   }
   wsync();
   APROF(AP_FORCES);
-  // per body B: the subtree sums T[B] = sum of fb[b] over the bodies b of B's subtree (54 floats each), a column per
-  // lane: lane c < 54 loads column c of every body and adds each body into its parent, highest id first (a body's id
+  // per body B: the subtree sums T[B] = sum of fb[b] over the bodies b of B's subtree (48 floats each), a column per
+  // lane: lane c < 48 loads column c of every body and adds each body into its parent, highest id first (a body's id
   // is above its parent's, so each body is complete when it is added), then stores the sums in place. The tree is
   // compile-time: 29 adds a lane, no masks. Lanes past the columns compute a copy of the last one and do not store.
   {
@@ -928,7 +954,10 @@ __device__ void adj_substep(Adj& s, const float* __restrict__ rec, int lane, int
     const int bj = j < 6 ? 1 : j - 4;
     const Sv F1 = ld_sv6(s.fb[bj][FB_F1]), P = ld_sv6(s.fb[bj][FB_P]), X1 = ld_sv6(s.fb[bj][FB_X1]);  // subtree sums
     const Sv F2 = ld_sv6(s.fb[bj][FB_F2]), P2 = ld_sv6(s.fb[bj][FB_P2]), EGs = ld_sv6(s.fb[bj][FB_EG]);
-    const Sv OLs = ld_sv6(s.fb[bj][FB_OL]), OAs = ld_sv6(s.fb[bj][FB_OA]), OVs = ld_sv6(s.fb[bj][FB_OV]);
+    const Sv OLs = ld_sv6(s.fb[bj][FB_OL]), OAs = ld_sv6(s.fb[bj][FB_OA]);
+    float kc, bc;  // the velocity cotangents' row sums are the damping b, one for every pair, times the accelerations'
+    kb_consts<aPSOLREF, aPSOLIMP>(&kc, &bc);
+    const Sv OVs = sv_add(sv0(), OAs, bc);
     Sv Vo = sv0(), Lo = sv0(), Yo = sv0(), Awo = sv0(), A1o = sv0(), A2o = sv0();
     for (int k = 0; k < 3; k++) A1o.v[k] = -kGrav[k];
     if (j >= 3 && j < 6) {

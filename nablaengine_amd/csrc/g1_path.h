@@ -66,6 +66,8 @@ constexpr LaneMask PATH_WAIST3 = lane_mask([](int g, int p) { return g == 3 && p
 template <int K>
 struct PathLt { static constexpr LaneMask m = lane_mask([](int, int p) { return p < K; }); };
 template <int K>
+struct PathGt { static constexpr LaneMask m = lane_mask([](int, int p) { return p > K; }); };
+template <int K>
 struct PathEq { static constexpr LaneMask m = lane_mask([](int, int p) { return p == K; }); };
 
 // the mask as a scalar register pair, built from opaque halves (scalar moves; no vector compare per use)
@@ -240,65 +242,133 @@ __device__ __forceinline__ void path_load(const float* buf, float (&c)[PP], int 
   for (int m = 0; m < PP; m++) c[m] = buf[m * PFS + lane];
 }
 
-// x = A^-1 b from path_factor's rows (in registers: c, and in buf) and diagonal; b on every lane of its dof (0 on the
-// lanes without one), x too. Each lane keeps its running value scaled by 1 / L[p][p], so the value broadcast at a step
-// is already the solved entry. L' y = b leaf first: the limbs (row 2's arm, row 3's arm and both legs at once); the
-// waist's and the root's dofs then take the right arm's terms, the left arm's, the waist's, the right leg's and the left
-// leg's, their running values handed from row to row. L x = y root first, lane p reading row p of L (the transposed
-// read of buf), each row alone. 49 steps of one multiply-add on the dependency chain and 30 coefficient products,
-// where the solve one dof at a time took 68 steps of four instructions; bitwise its result.
+// x = A^-1 b for N right-hand sides at once, A = L' L with the tree's sparsity: cf[m] = -L[m][p] / L[p][p] on the lanes
+// p < m (row m of lane p's path), l[k] = -L[p][k] / L[p][p] on the lanes p > k, 0 on the others; dself = 1 / L[p][p], 0 on
+// the lanes without a dof; b on every lane of its dof (0 on the lanes without one), x too. Each lane keeps its running
+// value scaled by 1 / L[p][p], so the value broadcast at a step is already the solved entry. L' y = b leaf first: the
+// limbs (row 2's arm, row 3's arm and both legs at once); the waist's and the root's dofs then take the right arm's
+// terms, the left arm's, the waist's, the right leg's and the left leg's, their running values handed from row to row. L x
+// = y root first, lane p along row p of L, each row alone. 49 steps of one multiply-add on the dependency chain, where
+// the solve one dof at a time takes 68 steps of four instructions; bitwise its result.
+template <int N>
+__device__ __forceinline__ void path_solve_scaled(const float (&cf)[PP], const float (&l)[PP], float dself,
+                                                  const float* b, float* x) {
+  float z[N], acc[N], o0, o1;
+#pragma unroll
+  for (int i = 0; i < N; i++) z[i] = b[i] * dself;
+  // one step z += (lane k's z) n on each chain; between a chain's steps two wait states, one of them the other chain's
+#define G1_ONE(k, n) G1_FMAC_BC("%0", "%0", n, k) G1_NOP
+#define G1_TWO(k, n) G1_FMAC_BC("%0", "%0", n, k) G1_FMAC_BC("%1", "%1", n, k) "s_nop 0\n\t"
+#define G1_ADD1(k, n) G1_FMAC_BC("%0", "%1", n, k)
+#define G1_ADD2(k, n) G1_FMAC_BC("%0", "%2", n, k) G1_FMAC_BC("%1", "%3", n, k)
+#define G1_BOTH(ONE, TWO, IN)                                                                                      \
+  if constexpr (N == 1) asm(G1_NOP ONE : "+v"(z[0]) : IN);                                                         \
+  else asm(G1_NOP TWO "s_nop 0" : "+v"(z[0]), "+v"(z[N - 1]) : IN);
+#define G1_ACC(ONE, TWO, IN)                                                                                       \
+  if constexpr (N == 1) asm(G1_NOP ONE "s_nop 1" : "+v"(acc[0]) : "v"(z[0]), IN);                                  \
+  else asm(G1_NOP TWO "s_nop 1" : "+v"(acc[0]), "+v"(acc[N - 1]) : "v"(z[0]), "v"(z[N - 1]), IN);
+#define G1_IN(...) __VA_ARGS__
+  G1_BOTH(G1_ONE(15, "%1") G1_ONE(14, "%2") G1_ONE(13, "%3") G1_ONE(12, "%4") G1_ONE(11, "%5") G1_ONE(10, "%6")
+          G1_ONE(9, "%7"),
+          G1_TWO(15, "%2") G1_TWO(14, "%3") G1_TWO(13, "%4") G1_TWO(12, "%5") G1_TWO(11, "%6") G1_TWO(10, "%7")
+          G1_TWO(9, "%8"),
+          G1_IN("v"(cf[15]), "v"(cf[14]), "v"(cf[13]), "v"(cf[12]), "v"(cf[11]), "v"(cf[10]), "v"(cf[9])))
+#pragma unroll
+  for (int i = 0; i < N; i++) row_pairs(z[i], &o0, &acc[i]);  // row 2's shared dofs go on from row 3's
+  G1_ACC(G1_ADD1(15, "%2") G1_ADD1(14, "%3") G1_ADD1(13, "%4") G1_ADD1(12, "%5") G1_ADD1(11, "%6") G1_ADD1(10, "%7")
+         G1_ADD1(9, "%8"),
+         G1_ADD2(15, "%4") G1_ADD2(14, "%5") G1_ADD2(13, "%6") G1_ADD2(12, "%7") G1_ADD2(11, "%8") G1_ADD2(10, "%9")
+         G1_ADD2(9, "%10"),
+         G1_IN("v"(cf[15]), "v"(cf[14]), "v"(cf[13]), "v"(cf[12]), "v"(cf[11]), "v"(cf[10]), "v"(cf[9])))
+#pragma unroll
+  for (int i = 0; i < N; i++) z[i] = lane_sel<PATH_SHARED2>(acc[i], z[i]);
+  G1_BOTH(G1_ONE(8, "%1") G1_ONE(7, "%2") G1_ONE(6, "%3"), G1_TWO(8, "%2") G1_TWO(7, "%3") G1_TWO(6, "%4"),
+          G1_IN("v"(cf[8]), "v"(cf[7]), "v"(cf[6])))
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    row_halves(z[i], &o0, &o1);  // row 2's root on to rows 0 and 1
+    row_pairs(o1, &acc[i], &o0);
+  }
+#define G1_LEGS                                                                                                    \
+  G1_ACC(G1_ADD1(11, "%2") G1_ADD1(10, "%3") G1_ADD1(9, "%4") G1_ADD1(8, "%5") G1_ADD1(7, "%6") G1_ADD1(6, "%7"),  \
+         G1_ADD2(11, "%4") G1_ADD2(10, "%5") G1_ADD2(9, "%6") G1_ADD2(8, "%7") G1_ADD2(7, "%8") G1_ADD2(6, "%9"),  \
+         G1_IN("v"(cf[11]), "v"(cf[10]), "v"(cf[9]), "v"(cf[8]), "v"(cf[7]), "v"(cf[6])))
+  G1_LEGS  // the right leg's terms (row 1)
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    row_pairs(acc[i], &o0, &o1);
+    acc[i] = o1;
+  }
+  G1_LEGS  // the left leg's (row 0)
+#undef G1_LEGS
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    row_pairs(acc[i], &o0, &o1);
+    row_halves(o0, &acc[i], &o1);  // row 0's root in every row; row 2's waist also in row 3
+    row_pairs(z[i], &o0, &o1);
+    z[i] = lane_sel<PATH_WAIST3>(o0, z[i]);
+    z[i] = lane_sel<PATH_ROOT>(acc[i], z[i]);
+  }
+  G1_BOTH(G1_ONE(5, "%1") G1_ONE(4, "%2") G1_ONE(3, "%3") G1_ONE(2, "%4") G1_ONE(1, "%5"),
+          G1_TWO(5, "%2") G1_TWO(4, "%3") G1_TWO(3, "%4") G1_TWO(2, "%5") G1_TWO(1, "%6"),
+          G1_IN("v"(cf[5]), "v"(cf[4]), "v"(cf[3]), "v"(cf[2]), "v"(cf[1])))
+#pragma unroll
+  for (int i = 0; i < N; i++) z[i] *= dself;
+  G1_BOTH(G1_ONE(0, "%1") G1_ONE(1, "%2") G1_ONE(2, "%3") G1_ONE(3, "%4") G1_ONE(4, "%5") G1_ONE(5, "%6")
+          G1_ONE(6, "%7") G1_ONE(7, "%8") G1_ONE(8, "%9") G1_ONE(9, "%10") G1_ONE(10, "%11") G1_ONE(11, "%12")
+          G1_ONE(12, "%13") G1_ONE(13, "%14") G1_ONE(14, "%15"),
+          G1_TWO(0, "%2") G1_TWO(1, "%3") G1_TWO(2, "%4") G1_TWO(3, "%5") G1_TWO(4, "%6") G1_TWO(5, "%7")
+          G1_TWO(6, "%8") G1_TWO(7, "%9") G1_TWO(8, "%10") G1_TWO(9, "%11") G1_TWO(10, "%12") G1_TWO(11, "%13")
+          G1_TWO(12, "%14") G1_TWO(13, "%15") G1_TWO(14, "%16"),
+          G1_IN("v"(l[0]), "v"(l[1]), "v"(l[2]), "v"(l[3]), "v"(l[4]), "v"(l[5]), "v"(l[6]), "v"(l[7]), "v"(l[8]),
+                "v"(l[9]), "v"(l[10]), "v"(l[11]), "v"(l[12]), "v"(l[13]), "v"(l[14])))
+#undef G1_IN
+#undef G1_ACC
+#undef G1_BOTH
+#undef G1_ADD2
+#undef G1_ADD1
+#undef G1_TWO
+#undef G1_ONE
+#pragma unroll
+  for (int i = 0; i < N; i++) x[i] = z[i];
+}
+
+// from path_factor's rows (in registers: c, and in buf) and diagonal
 __device__ __forceinline__ float path_solve(const float* buf, const float (&c)[PP], float diag, float b, int lane_) {
   const int lane = opaque_lane(lane_);
-  float l[PP];
+  float l[PP], cf[PP], x;
   const float* row = buf + (lane & 15) * PFS + (lane & 48);
 #pragma unroll
   for (int k = 0; k < PP - 1; k++) l[k] = row[k];
   const float dself = lane_sel0<PATH_VALID>(1.f / diag), ds = -dself;
-  float cf[PP];
 #pragma unroll
   for (int m = 1; m < PP; m++) cf[m] = c[m] * ds;
-  float z = b * dself;
-#define G1_STEP(k, n) G1_FMAC_BC("%0", "%0", n, k) G1_NOP
-#define G1_ADD(k, n) G1_FMAC_BC("%0", "%1", n, k)
-  asm(G1_NOP G1_STEP(15, "%1") G1_STEP(14, "%2") G1_STEP(13, "%3") G1_STEP(12, "%4") G1_STEP(11, "%5")
-      G1_STEP(10, "%6") G1_STEP(9, "%7")
-      : "+v"(z) : "v"(cf[15]), "v"(cf[14]), "v"(cf[13]), "v"(cf[12]), "v"(cf[11]), "v"(cf[10]), "v"(cf[9]));
-  float even, acc;
-  row_pairs(z, &even, &acc);  // row 2's shared dofs go on from row 3's
-  asm(G1_NOP G1_ADD(15, "%2") G1_ADD(14, "%3") G1_ADD(13, "%4") G1_ADD(12, "%5") G1_ADD(11, "%6") G1_ADD(10, "%7")
-      G1_ADD(9, "%8")
-      : "+v"(acc) : "v"(z), "v"(cf[15]), "v"(cf[14]), "v"(cf[13]), "v"(cf[12]), "v"(cf[11]), "v"(cf[10]), "v"(cf[9]));
-  z = lane_sel<PATH_SHARED2>(acc, z);
-  asm(G1_NOP G1_STEP(8, "%1") G1_STEP(7, "%2") G1_STEP(6, "%3")
-      : "+v"(z) : "v"(cf[8]), "v"(cf[7]), "v"(cf[6]));
-  float low, odd;
-  row_halves(z, &low, &acc);  // row 2's root on to rows 0 and 1
-  row_pairs(acc, &acc, &odd);
-#define G1_LEGS                                                                                                    \
-  asm(G1_NOP G1_ADD(11, "%2") G1_ADD(10, "%3") G1_ADD(9, "%4") G1_ADD(8, "%5") G1_ADD(7, "%6") G1_ADD(6, "%7") "s_nop 1" \
-      : "+v"(acc) : "v"(z), "v"(cf[11]), "v"(cf[10]), "v"(cf[9]), "v"(cf[8]), "v"(cf[7]), "v"(cf[6]))
-  G1_LEGS;  // the right leg's terms (row 1)
-  row_pairs(acc, &even, &acc);
-  G1_LEGS;  // the left leg's (row 0)
-#undef G1_LEGS
-  row_pairs(acc, &acc, &odd);
-  row_halves(acc, &acc, &odd);  // row 0's root in every row; row 2's waist also in row 3
-  row_pairs(z, &even, &odd);
-  z = lane_sel<PATH_WAIST3>(even, z);
-  z = lane_sel<PATH_ROOT>(acc, z);
-  asm(G1_NOP G1_STEP(5, "%1") G1_STEP(4, "%2") G1_STEP(3, "%3") G1_STEP(2, "%4") G1_FMAC_BC("%0", "%0", "%5", 1)
-      : "+v"(z) : "v"(cf[5]), "v"(cf[4]), "v"(cf[3]), "v"(cf[2]), "v"(cf[1]));
 #pragma unroll
   for (int k = 0; k < PP - 1; k++) l[k] *= ds;
-  z *= dself;
-  asm(G1_NOP G1_STEP(0, "%1") G1_STEP(1, "%2") G1_STEP(2, "%3") G1_STEP(3, "%4") G1_STEP(4, "%5") G1_STEP(5, "%6")
-      G1_STEP(6, "%7") G1_STEP(7, "%8") G1_STEP(8, "%9") G1_STEP(9, "%10") G1_STEP(10, "%11") G1_STEP(11, "%12")
-      G1_STEP(12, "%13") G1_STEP(13, "%14") G1_FMAC_BC("%0", "%0", "%15", 14)
-      : "+v"(z) : "v"(l[0]), "v"(l[1]), "v"(l[2]), "v"(l[3]), "v"(l[4]), "v"(l[5]), "v"(l[6]), "v"(l[7]), "v"(l[8]),
-                  "v"(l[9]), "v"(l[10]), "v"(l[11]), "v"(l[12]), "v"(l[13]), "v"(l[14]));
-#undef G1_STEP
-#undef G1_ADD
-  return z;
+  path_solve_scaled<1>(cf, l, dself, &b, &x);
+  return x;
+}
+
+// from a packed factor (lower, TRI layout) of the tree's sparsity; Lp readable up to its word 34 * 35 / 2 + 70 (the
+// lanes without a dof read past the factor and drop it)
+template <int N>
+__device__ __forceinline__ void path_solve_packed(const float* Lp, int pd, int lane_, const float* b, float* x) {
+  const int lane = opaque_lane(lane_), g = lane >> 4, o6 = g < 2 ? 6 * g : 12, o9 = g < 3 ? 6 * g : 19;
+  // row m's dof is m + o: its packed row starts at tri(m) + m o + o (o + 1) / 2
+  const float *col = Lp + pd, *row = Lp + tri(pd, 0);
+  const float *c6 = col + o6 * (o6 + 1) / 2, *c9 = col + o9 * (o9 + 1) / 2, *r6 = row + o6, *r9 = row + o9;
+  const float dself = lane_sel0<PATH_VALID>(1.f / row[pd]), ds = -dself;
+  float cf[PP], l[PP];
+#pragma unroll
+  for (int m = 1; m < PP; m++) cf[m] = m < 6 ? col[tri(m, 0)] : m < 9 ? c6[m * o6 + tri(m, 0)] : c9[m * o9 + tri(m, 0)];
+#pragma unroll
+  for (int k = 0; k < PP - 1; k++) l[k] = (k < 6 ? row : k < 9 ? r6 : r9)[k];
+  static_for<0, PP, 1>([&](auto mc) {
+    constexpr int m = decltype(mc)::value;
+    if constexpr (m > 0) cf[m] = lane_sel0<PathLt<m>::m>(cf[m] * ds);
+    if constexpr (m < PP - 1) l[m] = lane_sel0<PathGt<m>::m>(l[m] * ds);
+  });
+  path_solve_scaled<N>(cf, l, dself, b, x);
 }
 
 }  // namespace g1k

@@ -84,3 +84,35 @@ def test_path_factors_vs_oracle(kind):
         assert info[same, 1].max() > 16 and (info[same, 1] % 4 != 0).any(), info
     if kind == "flight":
         assert (info[:, 2] == 0).sum() >= 4, info  # worlds without any row (a hand may touch the hip in the others)
+
+
+@pytest.mark.parametrize("kind", ["flight", "all", "waist", "one_foot", "tangled", "feet"])
+def test_path_solves_in_the_adjoint(kind):
+    """One substep's VJP (exact mode) on the same states, whose tapes hold factors of both kinds (the tree's sparsity,
+    solved in the path layout, and with contacts between robot bodies, solved dof by dof), and the same VJPs as pairs of
+    cotangent sets. Against the oracle's: the float32 IFT solves with H (condition 1e5 to 1e6) leave about 1e-4 at one
+    substep (median over the worlds; the suite's gate for one substep's gradients); sets bitwise the single calls."""
+    import torch
+    from nablaengine_amd import torch_ffi
+    B = 12
+    st = _states(kind, B)
+    args = [torch.from_numpy(st[k]).cuda() for k in KEYS]
+    tape = torch_ffi.forward(*args, iterations=50, substeps=1, tape=True)[4]
+    cots = [synthetic.cotangents(B, seed=5 + i) for i in range(3)]
+    cq, cv = (torch.from_numpy(np.stack(x)).cuda() for x in zip(*cots))
+    sets = torch_ffi._vjp_sets(tape, args[4], args[5], cq, cv, substeps=1, clamp_kv=1, normal=0)
+    for i in range(3):
+        one = torch_ffi.backward(tape, args[4], args[5], cq[i].contiguous(), cv[i].contiguous(), substeps=1, clamp_kv=1,
+                                 normal=0)
+        for a, b in zip(one, sets):
+            assert torch.equal(a, b[i])
+    s64 = {k: st[k].astype(np.float64) for k in KEYS}
+    ref = oracle.vjp(**s64, g_qpos=cots[2][0].astype(np.float64), g_qvel=cots[2][1].astype(np.float64), clamp_kv=1,
+                     normal=0, **{**oracle.ENGINE, "iterations": 50}, nsub=1)
+    got = [x.cpu().numpy().astype(np.float64) for x in one[:3]]
+    for name, a, b in zip(("qpos", "qvel", "ctrl"), got, ref):
+        if name == "qpos":
+            a, b = oracle.qpos_tangent(s64["qpos"], a), oracle.qpos_tangent(s64["qpos"], b)
+        e = np.linalg.norm(a - b, axis=1) / np.maximum(np.linalg.norm(b, axis=1), 1e-12)
+        print(kind, name, f"median {np.median(e):.2g} max {e.max():.2g}")
+        assert np.isfinite(a).all() and (kind == "feet" or np.median(e) <= 1e-4), (name, e)
