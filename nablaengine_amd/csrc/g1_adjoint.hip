@@ -1086,10 +1086,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                                                 float* __restrict__ gctrl, int* __restrict__ info,
                                                 const float* __restrict__ ctrl, float clamp_soft, int clamp_kv,
                                                 int normal, const int* __restrict__ perm,
-                                                unsigned long long* __restrict__ diag, int ncot) {
+                                                unsigned long long* __restrict__ diag, int ncot, EarlyRange early) {
   __shared__ Adj s;
   const int lane = threadIdx.x;
   if ((int)blockIdx.x >= nw * ncot) return;
+  if ((int)blockIdx.x >= early.from && (int)blockIdx.x < early.to) __builtin_amdgcn_s_setprio(3);  // early_worlds
   // ncot sets of output cotangents on one tape, set-major: workgroup b takes set b / nw; within a set the worlds run
   // heaviest first (g1_order.hip). wr: the world's row in its set's cotangents, gradients and info
   const int kc = (int)blockIdx.x / nw, wi = (int)blockIdx.x - kc * nw;
@@ -1251,6 +1252,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 }
 
 int launch_order_adj(hipStream_t st, int nw, int nsub, const float* tape, void* work);
+EarlyRange early_worlds(int nw, int per_cu);
+constexpr int RESIDENT_PER_CU = 8;  // k_adjoint's worlds that a CU holds at once
 int resident_worlds();
 
 // k_adjoint_sets' sets per workgroup: groups small enough that nw x groups makes G1_SETS_WAVES waves, and at least
@@ -1283,7 +1286,7 @@ int launch_adjoint(hipStream_t st, int nw, int nsub, const float* tape, const fl
   }
   if (ncot == 1) {
     hipLaunchKernelGGL(k_adjoint, dim3(nw), dim3(64), 0, st, nw, nsub, tape, fric, com, gq_out, gv_out, gq_in, gv_in,
-                       gctrl, info, ctrl, clamp_soft, clamp_kv, normal, perm, diag, 1);
+                       gctrl, info, ctrl, clamp_soft, clamp_kv, normal, perm, diag, 1, early_worlds(nw, RESIDENT_PER_CU));
   } else {
     const int per = sets_per_group(nw, ncot), ngrp = (ncot + per - 1) / per;
     hipLaunchKernelGGL(k_adjoint_sets, dim3(nw * ngrp), dim3(64), 0, st, nw, nsub, tape, fric, com, gq_out, gv_out,

@@ -15,6 +15,9 @@ using namespace g1t;
 
 constexpr int WL = 64;  // lanes per world: one wave64
 
+// The positions of a launch's order that a kernel runs at top issue priority from start to end (see early_worlds)
+struct EarlyRange { int from, to; };
+
 template <int N>
 constexpr Arr<int, N> to_int(const int (&a)[N]) {
   Arr<int, N> r{};

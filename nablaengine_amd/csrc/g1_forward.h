@@ -24,6 +24,7 @@ struct __align__(16) Sim {
   float fric;
   int ncon, ncon_raw, nlim, nefc, flags, niter;
   int dcnt;  // the records' flags counted over the substeps: refactored | not converged << 8 | singular << 16
+  int top;    // the world's priority: 0 at top throughout, else the highest level it takes by its remaining work
   int acost;  // the adjoint's dispatch cost summed over the substeps so far (taped forward)
   unsigned clampm[2];  // dofs whose actuator force is at its limit (tape)
 #ifdef G1_PROFILE

@@ -1196,9 +1196,10 @@ constexpr float PRIO_STEP = 4e5f;
 // one world left. Starting at level 0 held it behind that wave for a substep: 1.5% slower forward at 4096 worlds than
 // starting at 1, 2 or 3, which measured alike.
 constexpr int PRIO_START = 2;
-__device__ __forceinline__ void set_priority_by_remaining(unsigned long long t_start, int k, int nsub) {
+// top: the highest level (2 in a launch that keeps level 3 for its early worlds)
+__device__ __forceinline__ void set_priority_by_remaining(unsigned long long t_start, int k, int nsub, int top) {
   const float rem = (float)(__builtin_amdgcn_s_memtime() - t_start) * (float)(nsub - k) / (float)k;
-  if (rem > 3.f * PRIO_STEP) __builtin_amdgcn_s_setprio(3);
+  if (rem > 3.f * PRIO_STEP && top > 2) __builtin_amdgcn_s_setprio(3);
   else if (rem > 2.f * PRIO_STEP) __builtin_amdgcn_s_setprio(2);
   else if (rem > PRIO_STEP) __builtin_amdgcn_s_setprio(1);
   else __builtin_amdgcn_s_setprio(0);
@@ -1213,6 +1214,7 @@ struct ForwardArgs {
   float *ocon, *tape;
   const int* perm;
   unsigned long long* diag;
+  EarlyRange early;
 };
 
 // one world on this wave64 (a workgroup of 64 lanes)
@@ -1237,6 +1239,8 @@ __device__ __forceinline__ void forward_world(Sim& s, const ForwardArgs& A) {
   if (lane < NV) { s.qvel[lane] = iv; s.qacc[lane] = iw; }
   if (lane < NU) s.ctrl[lane] = iu;
   if (lane < 3) s.com[lane] = ic;
+  if (lane == 0)  // an early world, else the highest priority level by remaining work
+    s.top = (int)blockIdx.x >= A.early.from && (int)blockIdx.x < A.early.to ? 0 : A.early.to > 0 ? 2 : 3;
   if (lane == 0) { s.fric = ifr; s.flags = 0; s.niter = 0; s.dcnt = 0; s.acost = 0; }
   s.dsub[lane] = lane < NV ? cTree.dofmask32[lane] : 0u;
   if (lane < 8) s.S[NV][lane] = 0.f;
@@ -1252,7 +1256,9 @@ __device__ __forceinline__ void forward_world(Sim& s, const ForwardArgs& A) {
   wsync();
   const unsigned long long t_start = __builtin_amdgcn_s_memtime();
   for (int k = 0; k < nsub; k++) {
-    if (k > 0) set_priority_by_remaining(t_start, k, nsub);
+    const int top = rdli(s.top, 0);  // (from LDS: held in a register through the substeps it cost 3%)
+    if (top == 0) __builtin_amdgcn_s_setprio(3);
+    else if (k > 0) set_priority_by_remaining(t_start, k, nsub, top);
     else __builtin_amdgcn_s_setprio(PRIO_START);
     substep(s, lane, iterations, tape ? tape + ((size_t)w * nsub + k) * REC_WORDS : nullptr,
             ocon && k == nsub - 1 ? ocon + (size_t)w * MAXCON * 8 : nullptr);
@@ -1304,12 +1310,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void
   forward_world(s, A);
 }
 constexpr int WAVES3_WORLDS_PER_CU = 9;  // beyond so many worlds a CU: k_forward3
+constexpr int RESIDENT2_PER_CU = 8, RESIDENT3_PER_CU = 11;  // worlds of either build that a CU holds at once
 
 }  // namespace g1k
 
 namespace g1k {
 int launch_order_fwd(hipStream_t st, int nw, const float* qpos, void* work);
 int worlds_of_cus(int per_cu);
+EarlyRange early_worlds(int nw, int per_cu);
 int resident_worlds();
 // order: 0 index order (work unused), 1 compute the order into work first (index order when the batch fits the
 // GPU's resident slots at once: the order cannot change the makespan there), 2 the order already in work; diag: the
@@ -1327,8 +1335,10 @@ int launch_forward(hipStream_t st, int nw, const float* qpos, const float* qvel,
     }
     perm = (const int*)work;
   }
-  const ForwardArgs A{nw, qpos, qvel, warm, ctrl, fric, com, iterations, nsub, oq, ov, ow, info, ocon, tape, perm, diag};
-  if (nw > worlds_of_cus(WAVES3_WORLDS_PER_CU)) hipLaunchKernelGGL(k_forward3, dim3(nw), dim3(64), 0, st, A);
+  const bool three = nw > worlds_of_cus(WAVES3_WORLDS_PER_CU);
+  const ForwardArgs A{nw,  qpos, qvel, warm, ctrl, fric, com,  iterations, nsub, oq, ov, ow, info, ocon, tape, perm,
+                      diag, early_worlds(nw, three ? RESIDENT3_PER_CU : RESIDENT2_PER_CU)};
+  if (three) hipLaunchKernelGGL(k_forward3, dim3(nw), dim3(64), 0, st, A);
   else hipLaunchKernelGGL(k_forward, dim3(nw), dim3(64), 0, st, A);
   return (int)hipGetLastError();
 }

@@ -46,6 +46,21 @@ int worlds_of_cus(int per_cu) {
 // when the CU count is not known (the order is then always computed)
 int resident_worlds() { return worlds_of_cus(WORLDS_PER_CU); }
 
+// A launch of more worlds than are resident at once (R = per_cu a CU) and fewer than twice as many: its second round is
+// the last. Were the worlds that share a SIMD to advance alike, they would end together, and a second-round world
+// would then run through by itself, at about half the rate the SIMD has with its slots full. So the last E of the
+// first round's positions (the order's lightest there) run at top priority and end early, and their successors run beside
+// the heavier worlds from then on. E = the second round's worlds, at most 4 a CU, and fewer as the second round fills up
+// (the SIMDs are then full to its end anyway). Forward of standing / contact-heavy worlds in us, without and with:
+// 3072 521 / 560 and 520 / 556, 3584 599 / 661 and 587 / 625, 4096 677 / 738 and 626 / 678, 5000 747 / 818 and 726 / 804;
+// VJP of 2560 worlds 114 / 124 and 106 / 116, of 3000 121 / 132 and 112 / 122, of 4096 the same.
+EarlyRange early_worlds(int nw, int per_cu) {
+  const int R = worlds_of_cus(per_cu), four = worlds_of_cus(4);
+  int e = nw - R < 2 * R - nw ? nw - R : 2 * R - nw;
+  if (e > four) e = four;
+  return e > 0 ? EarlyRange{R - e, R} : EarlyRange{0, 0};
+}
+
 // contacts at the input state: FK of body poses (each body lane walks its chain from the root), geom poses, the main
 // kernel's broadphase and narrowphase (the same code); the cost counts the contacts' constraint rows (4 per pyramid
 // contact, 1 per frictionless one) plus a weight per contact between two robot bodies (each makes the Newton Hessian
