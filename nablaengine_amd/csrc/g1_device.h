@@ -33,9 +33,7 @@ __constant__ inline Arr<float, NB * 3> cIpos = to_float(BODY_IPOS);
 __constant__ inline Arr<float, NB * 4> cIquat = to_float(BODY_IQUAT);
 __constant__ inline Arr<float, NB> cMass = to_float(BODY_MASS);
 __constant__ inline Arr<float, NB * 3> cInert = to_float(BODY_INERTIA);
-__constant__ inline Arr<int, NB> cParent = to_int(BODY_PARENT);
 __constant__ inline Arr<int, NB> cDepth = to_int(BODY_DEPTH);
-__constant__ inline Arr<int, NB> cQadr = to_int(BODY_QADR);
 __constant__ inline Arr<float, NV> cArm = to_float(DOF_ARMATURE);
 __constant__ inline Arr<float, NV> cDinvw = to_float(DOF_INVWEIGHT0);
 __constant__ inline Arr<float, NV> cKp = to_float(DOF_KP);
