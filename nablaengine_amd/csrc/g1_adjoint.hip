@@ -1256,17 +1256,24 @@ EarlyRange early_worlds(int nw, int per_cu);
 constexpr int RESIDENT_PER_CU = 8;  // k_adjoint's worlds that a CU holds at once
 int resident_worlds();
 
-// k_adjoint_sets' sets per workgroup: groups small enough that nw x groups makes G1_SETS_WAVES waves, and at least
-// two groups (a workgroup of all of a world's sets is a long wave, whose tail shows at 16384 worlds: 1.3% there).
-// Of 2048 resident waves (2 per SIMD on 256 CUs), 16384 makes 8 rounds: the launch's tail is a few sets long, and the
-// record phases repeated per group cost under 2% (measured at 1024, 4096 and 16384 worlds with 4096 to 32768 waves:
-// 16384 the best at 4096 worlds and within 0.5% at 1024)
-#ifndef G1_SETS_WAVES
-#define G1_SETS_WAVES 16384
-#endif
+// k_adjoint_sets' sets per workgroup. A workgroup pays the tape's phases once and takes its sets in pairs (a last odd
+// one costs nearly a pair's solves), so larger groups do less work; smaller ones leave a shorter tail. Groups small
+// enough that nw x groups makes SETS_WAVES waves (8 rounds of the 2048 resident ones: a tail of a few sets), an even
+// number of sets each, at least two groups a world (one group of all sets is 1.3% slower at 16384 worlds). us for 71
+// sets, the odd group that the wave count alone gives and the even one: 500 worlds 3 939, 4 903; 600 3 1084, 4 1042;
+// 700 3 1269, 4 1218; 1000 5 1721, 6 1675; other even sizes are within 1% or slower from 250 to 16384 worlds.
+// Where that makes a group of one set, the launch is a few rounds long and whole rounds count: a pair's workgroup takes
+// 1.6 times a single set's (94 and 59 us alone), so the fewer weighted rounds win. Single sets / pairs: 28 worlds 87 /
+// 111, 40 144 / 131, 56 158 / 130, 60 184 / 196, 72 203 / 207, 100 262 / 231, 160 404 / 354, 200 485 / 431.
+constexpr long long SETS_WAVES = 16384;
 int sets_per_group(int nw, int ncot) {
-  const long long ngrp = std::min<long long>(ncot, std::max<long long>(2, (G1_SETS_WAVES + nw - 1) / nw));
-  return (int)((ncot + ngrp - 1) / ngrp);
+  const long long ngrp = std::min<long long>(ncot, std::max<long long>(2, (SETS_WAVES + nw - 1) / nw));
+  const int per = (int)((ncot + ngrp - 1) / ngrp);
+  if (per > 1) return std::min(ncot, per + per % 2);
+  const long long r = resident_worlds();
+  if (r <= 0) return 1;
+  const long long single = ((long long)nw * ncot + r - 1) / r, pairs = ((long long)nw * ((ncot + 1) / 2) + r - 1) / r;
+  return 10 * single <= 16 * pairs ? 1 : 2;
 }
 int launch_adjoint(hipStream_t st, int nw, int nsub, const float* tape, const float* fric, const float* com,
                    const float* gq_out, const float* gv_out, float* gq_in, float* gv_in, float* gctrl, int* info,
