@@ -158,13 +158,36 @@ __device__ __forceinline__ void path_products(float (&c)[PP], const float (&base
 constexpr int PFS = 65;
 constexpr int PATH_FACTOR_WORDS = PP * PFS;
 
-template <int M0, int N>  // c[m] -= (lane m's u) u for m = M0 + N - 1 .. M0
-__device__ __forceinline__ void path_update(float (&c)[PP], float u) {
-  if constexpr (N >= 1) {
-    constexpr int m = M0 + N - 1;
-    asm("v_fmac_f32_dpp %0, %1, -%1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "+v"(c[m]) : "v"(u), "n"(m));
-    path_update<M0, N - 1>(c, u);
-  }
+// c[m] -= (lane m's u) u for m = M0 .. M0 + N - 1, in one block that opens with the wait states (a block per row behind a
+// wait of its own would leave the compiler room for a register copy in between). u passes through it, so what reads u by
+// a lane swap next has waited too (N = 0: the wait alone).
+template <int M0, int N>
+__device__ __forceinline__ void path_update(float (&c)[PP], float& u) {
+  static_assert(N >= 0 && N <= 6 && M0 + N <= PP, "path_update's rows");
+#define G1_U(acc, u, k) "v_fmac_f32_dpp %" #acc ", %" #u ", -%" #u " row_newbcast:%" #k " row_mask:0xf bank_mask:0xf\n\t"
+  float* const r = c + M0;
+  if constexpr (N == 0)
+    asm("s_nop 1" : "+v"(u));
+  else if constexpr (N == 1)
+    asm(G1_NOP G1_U(0, 1, 2) : "+v"(r[0]), "+v"(u) : "n"(M0));
+  else if constexpr (N == 2)
+    asm(G1_NOP G1_U(1, 2, 4) G1_U(0, 2, 3) : "+v"(r[0]), "+v"(r[1]), "+v"(u) : "n"(M0), "n"(M0 + 1));
+  else if constexpr (N == 3)
+    asm(G1_NOP G1_U(2, 3, 6) G1_U(1, 3, 5) G1_U(0, 3, 4)
+        : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(u) : "n"(M0), "n"(M0 + 1), "n"(M0 + 2));
+  else if constexpr (N == 4)
+    asm(G1_NOP G1_U(3, 4, 8) G1_U(2, 4, 7) G1_U(1, 4, 6) G1_U(0, 4, 5)
+        : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(u)
+        : "n"(M0), "n"(M0 + 1), "n"(M0 + 2), "n"(M0 + 3));
+  else if constexpr (N == 5)
+    asm(G1_NOP G1_U(4, 5, 10) G1_U(3, 5, 9) G1_U(2, 5, 8) G1_U(1, 5, 7) G1_U(0, 5, 6)
+        : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(u)
+        : "n"(M0), "n"(M0 + 1), "n"(M0 + 2), "n"(M0 + 3), "n"(M0 + 4));
+  else if constexpr (N == 6)
+    asm(G1_NOP G1_U(5, 6, 12) G1_U(4, 6, 11) G1_U(3, 6, 10) G1_U(2, 6, 9) G1_U(1, 6, 8) G1_U(0, 6, 7)
+        : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(u)
+        : "n"(M0), "n"(M0 + 1), "n"(M0 + 2), "n"(M0 + 3), "n"(M0 + 4), "n"(M0 + 5));
+#undef G1_U
 }
 
 // A = L' L, eliminated leaf first (the tree's sparsity, no fill): lane p's c[m] (m >= p) is A[m][p] of its path (the
@@ -214,7 +237,9 @@ __device__ __forceinline__ float path_factor(float (&c)[PP], float* buf, int lan
     const float row = c[k] * rs;
     diag = lane_sel<PathEq<k>::m>(row, diag);
     float u = lane_sel0<PathLt<k>::m>(row);
-    asm("s_nop 1" : "+v"(u));  // read by DPP and by the row swap next
+    if constexpr (k >= 9) path_update<9, k - 9>(c, u);
+    else if constexpr (k > 6) path_update<6, k - 6>(c, u);
+    else if constexpr (k > 0 && k < 6) path_update<0, k>(c, u);
     c[k] = u;
     if constexpr (k >= 9) {
       float l, r;
@@ -224,11 +249,6 @@ __device__ __forceinline__ float path_factor(float (&c)[PP], float* buf, int lan
           "v_fmac_f32_dpp %2, %3, -%3" G1_BC(8) "v_fmac_f32_dpp %0, %4, -%4" G1_BC(6) "v_fmac_f32_dpp %1, %4, -%4" G1_BC(7)
           "v_fmac_f32_dpp %2, %4, -%4" G1_BC(8)
           : "+v"(c[6]), "+v"(c[7]), "+v"(c[8]) : "v"(a), "v"(b));
-      path_update<9, k - 9>(c, u);
-    } else if constexpr (k >= 6) {
-      path_update<6, k - 6>(c, u);
-    } else {
-      path_update<0, k>(c, u);
     }
   });
   float* st = buf + lane;
