@@ -1259,19 +1259,26 @@ int resident_worlds();
 // k_adjoint_sets' sets per workgroup. A workgroup pays the tape's phases once and takes its sets in pairs (a last odd
 // one costs nearly a pair's solves), so larger groups do less work; smaller ones leave a shorter tail. Groups small
 // enough that nw x groups makes SETS_WAVES waves (8 rounds of the 2048 resident ones: a tail of a few sets), an even
-// number of sets each, at least two groups a world (one group of all sets is 1.3% slower at 16384 worlds). us for 71
-// sets, the odd group that the wave count alone gives and the even one: 500 worlds 3 939, 4 903; 600 3 1084, 4 1042;
+// number of sets each; 3 sets and more make at least two groups (one group of 71 is 1.3% slower at 16384 worlds). us for
+// 71 sets, the odd group that the wave count alone gives and the even one: 500 worlds 3 939, 4 903; 600 3 1084, 4 1042;
 // 700 3 1269, 4 1218; 1000 5 1721, 6 1675; other even sizes are within 1% or slower from 250 to 16384 worlds.
-// Where that makes a group of one set, the launch is a few rounds long and whole rounds count: a pair's workgroup takes
-// 1.6 times a single set's (94 and 59 us alone), so the fewer weighted rounds win. Single sets / pairs: 28 worlds 87 /
-// 111, 40 144 / 131, 56 158 / 130, 60 184 / 196, 72 203 / 207, 100 262 / 231, 160 404 / 354, 200 485 / 431.
+// Where that makes a group of one set (few worlds, or few sets of any number of worlds) the choice is single sets or
+// pairs. A pair's workgroup takes 1.6 times a single set's (94 and 59 us alone), so the fewer weighted rounds win, a last
+// odd set counted as a pair. Single sets / pairs, worlds x sets: 40 x 71 144 / 131, 56 x 71 158 / 130, 60 x 71 184 / 196,
+// 72 x 71 203 / 207, 100 x 71 262 / 231, 200 x 71 485 / 431; 2000 x 2 155 / 150, 1000 x 4 168 / 150, 4096 x 2 283 / 234,
+// 16384 x 2 1089 / 861, 4096 x 4 532 / 431. (For 3 and 5 sets the odd one's count is too high: 1500 x 3 186 / 164,
+// 4096 x 3 406 / 353 run as single sets.)
+// Single sets just past one round are the exception: when the waves past it are all of the last set (its lightest
+// worlds) and at most 3/8 of a round, that second round is short. Single sets / pairs, and what the weighted rounds
+// alone would pick: 29 x 71 109 / 135, 1100 x 2 121 / 147, 1280 x 2 130 / 150, 1300 x 2 130 / 158, 1400 x 2 134 / 145,
+// 900 x 3 138 / 145, 600 x 4 127 / 142, 400 x 6 128 / 138: pairs. Past it: 32 x 71 143 / 134, 700 x 4 144 / 141.
 constexpr long long SETS_WAVES = 16384;
 int sets_per_group(int nw, int ncot) {
   const long long ngrp = std::min<long long>(ncot, std::max<long long>(2, (SETS_WAVES + nw - 1) / nw));
   const int per = (int)((ncot + ngrp - 1) / ngrp);
   if (per > 1) return std::min(ncot, per + per % 2);
-  const long long r = resident_worlds();
-  if (r <= 0) return 1;
+  const long long r = resident_worlds(), over = (long long)nw * ncot - r;
+  if (r <= 0 || (over <= nw && 8 * over <= 3 * r)) return 1;
   const long long single = ((long long)nw * ncot + r - 1) / r, pairs = ((long long)nw * ((ncot + 1) / 2) + r - 1) / r;
   return 10 * single <= 16 * pairs ? 1 : 2;
 }
