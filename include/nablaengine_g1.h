@@ -18,7 +18,7 @@ extern "C" {
  * tape (nw, nsub * DK_REC_WORDS) or NULL: the adjoint's record (its flags word as the reference's: 4 / 16
  * overflow, 1 << 8 refactored at the final zones, 1 << 9 not converged, 1 << 10 near-singular self contact); work:
  * dk_fwd_work_bytes(nw) bytes or NULL when 0, for the dispatch order (heaviest worlds first), which is skipped, and work
- * left unwritten, when the GPU holds all nw worlds at once (8 per CU): every world then starts at the launch. */
+ * left unwritten, up to 8 worlds per CU: the GPU then holds them all at once. */
 int dk_fwd_forward(hipStream_t st, int nw, const float* qpos, const float* qvel, const float* warm, const float* ctrl,
                    const float* fric, const float* com, int iterations, int nsub, float* oq, float* ov, float* ow,
                    int* info, float* ocon, float* tape, void* work);
@@ -35,7 +35,8 @@ int dk_fwd_forward_ordered(hipStream_t st, int nw, const float* qpos, const floa
  * arguments without work, and the same results; the dispatch order lives in a static device array of the library
  * (1 MiB per GPU, held until the process ends) whose address dk_fwd_upload takes once per device (else the first
  * call on the device does). At most DK_STATIC_MAX_WORLDS worlds: more returns DK_ERR_STATIC_CAPACITY without a
- * launch. Nothing is allocated. Every call on one GPU shares that array, so calls that overlap on one GPU (two
+ * launch. Nothing is allocated, but for the scratch memory that the HIP runtime sets up when a process first launches the
+ * forward of more than 9 worlds per CU (make such a call at set-up). Every call on one GPU shares that array, so calls that overlap on one GPU (two
  * streams at once) race; calls in one stream's order do not. */
 #define DK_STATIC_MAX_WORLDS 131072
 #define DK_ERR_STATIC_CAPACITY (-2)

@@ -601,7 +601,8 @@ struct __align__(16) SetStage { float vt[36], qn[36], y[36], lam[36], ub[32]; };
 constexpr int SET_CHUNK = 2;  // cotangent sets whose solves run together (two right-hand sides a pass)
 
 // adj_solves for the staged sets st[0 .. nc) at once (nc <= 2): the same expressions for each set, the pair of
-// right-hand sides through ltl_solve2, so each set's y and lambda are bitwise adj_solves' for it
+// right-hand sides through path_solve_packed<2>, or ltl_solve2 for an L_H with contacts between robot bodies, so each
+// set's y and lambda are bitwise adj_solves' for it
 __device__ __forceinline__ void adj_solves_sets(Adj& s, SetStage* st, int nc, int lane, bool clear) {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the factors' copies have landed in LDS
   wsync();
@@ -1262,8 +1263,8 @@ int resident_worlds();
 // number of sets each; 3 sets and more make at least two groups (one group of 71 is 1.3% slower at 16384 worlds). us for
 // 71 sets, the odd group that the wave count alone gives and the even one: 500 worlds 3 939, 4 903; 600 3 1084, 4 1042;
 // 700 3 1269, 4 1218; 1000 5 1721, 6 1675; other even sizes are within 1% or slower from 250 to 16384 worlds.
-// Where that makes a group of one set (few worlds, or few sets of any number of worlds) the choice is single sets or
-// pairs. A pair's workgroup takes 1.6 times a single set's (94 and 59 us alone), so the fewer weighted rounds win, a last
+// Where that makes a group of one set (few worlds or few sets: 71 of up to 230 worlds, 3 of up to 8191, 2 of any number)
+// the choice is single sets or pairs. A pair's workgroup takes 1.6 times a single set's (94 and 59 us alone), so the fewer weighted rounds win, a last
 // odd set counted as a pair. Single sets / pairs, worlds x sets: 40 x 71 144 / 131, 56 x 71 158 / 130, 60 x 71 184 / 196,
 // 72 x 71 203 / 207, 100 x 71 262 / 231, 200 x 71 485 / 431; 2000 x 2 155 / 150, 1000 x 4 168 / 150, 4096 x 2 283 / 234,
 // 16384 x 2 1089 / 861, 4096 x 4 532 / 431. (For 3 and 5 sets the odd one's count is too high: 1500 x 3 186 / 164,
@@ -1289,7 +1290,7 @@ int launch_adjoint(hipStream_t st, int nw, int nsub, const float* tape, const fl
   if (nw <= 0) return 0;
   if (reinterpret_cast<uintptr_t>(tape) & 15u) return (int)hipErrorInvalidValue;  // 16-byte copies of the factors
   const int* perm = nullptr;
-  // one set of a batch that fits the resident slots at once: every world starts at the launch, index order
+  // one set of a batch of up to 8 worlds per CU: index order (g1_order.hip)
   if (order == 1 && ncot == 1 && nw <= resident_worlds()) order = 0;
   if (work && order) {  // the dispatch order, heaviest worlds first (order 1: computed here; 2: already in work)
     if (order == 1) {

@@ -1,8 +1,8 @@
 // The G1 control step, forward: one wave64 per world, all substeps in one launch.
 //
 // Per substep (the reference's substep_pre / substep_post, g1_engine/step.py:1650-2184, restated for wave64):
-//   smooth     FK by each body walking its own chain (no level barriers), RNE bias and composite inertias by subtree
-//              masks, CRBA, clamped PD actuators, qacc_smooth = M^-1 qfrc_smooth (register Cholesky)
+//   smooth     FK by each body walking its own chain (no level barriers), RNE bias and composite inertias summed over
+//              subtrees a column per lane, CRBA, clamped PD actuators, qacc_smooth = M^-1 qfrc_smooth (g1_path.h)
 //   collision  geom poses, bounding-sphere broadphase over the 502 pairs (ballot compaction in pair order),
 //              narrowphase one candidate per lane, contacts compacted in (pair, slot) order by a wave prefix sum
 //   rows       limits on their dof's lane, contact rows (4 pyramid edges or 1 normal row) on the contact's lane, all
@@ -1183,18 +1183,18 @@ __device__ __forceinline__ void substep(Sim& s, int lane_, int iterations, float
   wsync();
 }
 
-// The wave's issue priority (s_setprio, 0..3; it changes which of a SIMD's two waves issues first, never a result)
+// The wave's issue priority (s_setprio, 0..3; it changes which of a SIMD's waves issues first, never a result)
 // from the cycles the world is expected still to need: its mean cycles per substep so far (s_memtime, the shader
 // clock) times the substeps left, one level per PRIO_STEP. The longest remaining work goes first, as the dispatch
 // order's heaviest-first does at launch: a world whose cost the launch's estimate missed (a self contact appearing
-// within the step, more Newton iterations) catches up on its co-resident light world instead of finishing last.
+// within the step, more Newton iterations) catches up on its co-resident light worlds instead of finishing last.
 // 4e5 cycles (about two mean substeps) was the best of 2e5 .. 1e6 at 4096 worlds, and 3e5 .. 4e5 again on the later
 // build with PRIO_START.
 constexpr float PRIO_STEP = 4e5f;
 // A world's level for its first substep, before it has a rate of its own: a world dispatched into the launch's second
-// round then has all its substeps left (at the mean rate about 2 PRIO_STEP), where its co-resident wave has part of
-// one world left. Starting at level 0 held it behind that wave for a substep: 1.5% slower forward at 4096 worlds than
-// starting at 1, 2 or 3, which measured alike.
+// round then has all its substeps left (at the mean rate about 2 PRIO_STEP), where its co-resident waves have part
+// of a world left. Starting at level 0 held it behind them for a substep: 1.5% slower forward at 4096 worlds (the
+// two-wave build) than starting at 1, 2 or 3, which measured alike.
 constexpr int PRIO_START = 2;
 // top: the highest level (2 in a launch that keeps level 3 for its early worlds)
 __device__ __forceinline__ void set_priority_by_remaining(unsigned long long t_start, int k, int nsub, int top) {
@@ -1295,10 +1295,10 @@ __device__ __forceinline__ void forward_world(Sim& s, const ForwardArgs& A) {
 }
 
 // Two builds of the kernel, the same results. k_forward: two waves per SIMD with registers to spare (190), the shortest
-// chain of a world by itself. k_forward3: three waves per SIMD (168 registers, 26 values in scratch, outside Newton's
-// loop but for a few loads; 14 KB of LDS, 11 worlds per CU): two waves leave a quarter of the SIMD's issue slots empty
-// (63 k VALU instructions a world-step in 168 k slots of its wave), the third fills them, and a world by itself takes 2%
-// longer. Forward of standing / contact-heavy worlds in us, two waves against three: 2048 550 / 508 against 563 / 516,
+// chain of a world by itself. k_forward3: three waves per SIMD (168 registers, 25 spilled to 80 B a lane of scratch,
+// outside Newton's loop but for a few loads; 14 KB of LDS, 11 worlds per CU): two waves leave a quarter of the SIMD's issue
+// slots empty (60.9 k VALU instructions a world-step in 159 k slots of its wave at 2304 worlds), the third fills them, and
+// a world by itself takes 2% longer. Forward of standing / contact-heavy worlds in us, two waves against three: 2048 550 / 508 against 563 / 516,
 // 2304 483 / 517 against 499 / 533, 2560 533 / 581 against 500 / 539, 3072 602 / 665 against 513 / 556, 4096 705 / 742
 // against 673 / 729, 16384 2353 / 2560 against 2000 / 2184: three waves from more than 9 worlds a CU on.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_forward(ForwardArgs A) {
@@ -1319,9 +1319,8 @@ int launch_order_fwd(hipStream_t st, int nw, const float* qpos, void* work);
 int worlds_of_cus(int per_cu);
 EarlyRange early_worlds(int nw, int per_cu);
 int resident_worlds();
-// order: 0 index order (work unused), 1 compute the order into work first (index order when the batch fits the
-// GPU's resident slots at once: the order cannot change the makespan there), 2 the order already in work; diag: the
-// diagnostic counters added to by each world at its end, or NULL
+// order: 0 index order (work unused), 1 compute the order into work first (index order up to 8 worlds per CU,
+// g1_order.hip), 2 the order already in work; diag: the diagnostic counters added to by each world at its end, or NULL
 int launch_forward(hipStream_t st, int nw, const float* qpos, const float* qvel, const float* warm, const float* ctrl,
                    const float* fric, const float* com, int iterations, int nsub, float* oq, float* ov, float* ow,
                    int* info, float* ocon, float* tape, void* work, int order, unsigned long long* diag) {

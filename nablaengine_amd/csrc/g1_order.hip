@@ -15,9 +15,15 @@
 // as blockIdx.x -> world. Results do not depend on the order: every world's computation is the same wherever and
 // whenever it runs, so the permutation only moves work in time (its order inside a bucket is free).
 //
-// A batch that fits the GPU's resident slots at once (8 worlds per CU in both kernels) starts every world at the
-// launch: no world waits for a slot, so the order cannot shorten the makespan, and the order's two launches are
-// skipped (index order).
+// A batch of up to 8 worlds per CU (what k_forward and k_adjoint hold at once) starts every world at the launch: no
+// world waits for a slot, and the order's two launches are skipped (index order). The order still decides which worlds
+// share a CU and its SIMDs. Forward in us, ordered against index order, 3 batches each, standing / contact-heavy worlds:
+//   512, 1024      4 to 13 slower / 10 to 14 slower (the two launches)
+//   1331           12 slower to 22 faster / 8 to 78 faster
+//   2048           5 slower to 20 faster / 4 to 20 faster
+//   2304           101 to 124 faster / 143 to 163 faster (k_forward: more worlds than it holds)
+//   2320 to 2816   8 slower to 46 faster / 2 slower to 79 faster (k_forward3: 11 worlds a CU, it holds them all)
+//   3000           76 to 105 faster / 95 to 135 faster
 #include <atomic>
 
 #include "g1_device.h"
@@ -42,8 +48,8 @@ int worlds_of_cus(int per_cu) {
   }
   return per_cu * cus;
 }
-// a batch up to this size is resident at once: 8 worlds per CU (two waves per SIMD, the adjoint's and k_forward's); 0
-// when the CU count is not known (the order is then always computed)
+// a batch up to this size runs in index order: 8 worlds per CU, resident at once in k_forward and k_adjoint (two waves
+// per SIMD); 0 when the CU count is not known (the order is then always computed)
 int resident_worlds() { return worlds_of_cus(WORLDS_PER_CU); }
 
 // A launch of more worlds than are resident at once (R = per_cu a CU) and fewer than twice as many: its second round is
@@ -54,6 +60,8 @@ int resident_worlds() { return worlds_of_cus(WORLDS_PER_CU); }
 // (the SIMDs are then full to its end anyway). Forward of standing / contact-heavy worlds in us, without and with:
 // 3072 521 / 560 and 520 / 556, 3584 599 / 661 and 587 / 625, 4096 677 / 738 and 626 / 678, 5000 747 / 818 and 726 / 804;
 // VJP of 2560 worlds 114 / 124 and 106 / 116, of 3000 121 / 132 and 112 / 122, of 4096 the same.
+// In index order (no work buffer) those positions hold any worlds: over batches of 2900 to 5400 worlds the forward then
+// takes 5% less to 4% more with them (0.5% less in the mean), the VJP of 2100 to 3400 4% less to 5% more (the same).
 EarlyRange early_worlds(int nw, int per_cu) {
   const int R = worlds_of_cus(per_cu), four = worlds_of_cus(4);
   int e = nw - R < 2 * R - nw ? nw - R : 2 * R - nw;

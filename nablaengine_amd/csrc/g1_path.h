@@ -12,7 +12,9 @@
 //
 // Every result is bitwise that of the dof-per-lane elimination and solves (each entry's updates are the same products
 // in the same order; where the limbs meet, at the waist and the root, the rows of lanes take their turns): the
-// factor's and the solver's rounding, and with it Newton's iteration counts, do not depend on the layout.
+// factor's and the solver's rounding, and with it Newton's iteration counts, do not depend on the layout. Compared: the
+// solves with a replay one dof at a time; states, info and tapes (both factors of every substep) of 24 batches of 1 to
+// 4096 worlds with the dof-per-lane build's.
 #pragma once
 #include "g1_device.h"
 
